@@ -167,3 +167,22 @@ def test_full_size_workload(device):
     print(f"hits {len(hit)}; FP32 t vs FP64: median rel err {np.median(rel):.2e}, "
           f"99.9th pct {np.quantile(rel, 0.999):.2e}, max {rel.max():.2e}")
     assert np.median(rel) < 1e-6 and np.quantile(rel, 0.999) < 1e-4
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 257, 16383, 16385, 2560 * 128 + 1])
+def test_ray_counts_around_waves_and_chunks(device, n):
+    """Ray counts at the edges of how a launch is divided: fewer rays than
+    waves, one more or less than a wave or a round of waves, and more chunks
+    than waves; every third ray is axis-parallel (an infinite inverse
+    direction) or has a component whose scaled inverse overflows.  The
+    oracle's brute force is exact, so equality is the bound."""
+    tris = V.gen_triangle_soup(150, seed=5, mu=-1.0, sigma=0.5)
+    _, o, d = scenes.soup(16, n, seed=n)
+    d = np.array(d, np.float32).reshape(-1, 3)
+    d[0::6] = [0, 0, -1]
+    d[3::6] = [1e-34, 1, -1e-36]
+    s, m = _scene(device, tris)
+    prim, t = s.intersect_closest(m, o, d)
+    bp, bt = _brute(tris, np.asarray(o).reshape(-1, 3), d)
+    assert np.array_equal(prim, bp)
+    assert np.array_equal(t.view(np.uint32), bt.view(np.uint32))

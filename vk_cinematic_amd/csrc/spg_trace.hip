@@ -1,8 +1,9 @@
 // gfx950 kernels of the wavefront path tracer.
 //
-//   closest hit   k_closest_mesh   one ray per lane, BVH2 with both child
-//                                  boxes per 64-byte node, LDS stack, t-max
-//                                  culling, strict-FP slab and MT tests
+//   closest hit   k_closest_mesh   one ray per lane, four-wide 64-byte
+//                                  nodes, one kind of step per iteration,
+//                                  LDS stack, t-max culling, strict-FP
+//                                  slab and MT tests
 //   scene query   k_intersect_scene  TLAS over instances -> per-instance
 //                                  local ray -> BLAS (sp_RayIntersectScene)
 //   wavefront     k_raygen -> (k_extend -> k_shade)* -> k_finalize
@@ -623,7 +624,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_intersect_scene(
     uint32_t rays = 0;
     SceneView sv = scene_view(S);
     auto begin = [&](uint32_t i, Trav &s) {
-        trav_begin_scene(s, v3{rays6[6 * i], rays6[6 * i + 1], rays6[6 * i + 2]},
+        trav_begin_scene(sv, s, v3{rays6[6 * i], rays6[6 * i + 1], rays6[6 * i + 2]},
                          v3{rays6[6 * i + 3], rays6[6 * i + 4], rays6[6 * i + 5]});
         return S.instCount > 0;
     };
@@ -739,11 +740,11 @@ __global__ __launch_bounds__(256) void k_raygen(TraceParams p)
     }
 }
 
-// Closest hit of every queued ray.  (Forcing a register budget of 6, 7 or
-// 8 resident waves per SIMD instead of the 5 that 84 registers give was
-// measured slower on the 4M-triangle box scene: 1.44, 1.80 and 2.43 ms per
-// launch against 1.41; the step is bound by instruction issue, and 7 and 8
-// spill.)
+// Closest hit of every queued ray, bound by vector instruction issue and, on
+// scenes beyond the L2, by the latency of the node fetches.  (A register
+// budget of 6 resident waves per SIMD instead of the 5 that the kernel's
+// registers give is slower: more waves evict each other's nodes from the
+// CU's L1.)
 // kShadow: the shadow rays of next-event estimation (queue 2).  A ray
 // toward the sky only asks whether anything is hit, so it stops at the
 // first instance with a hit; a ray toward an emissive triangle starts with
@@ -769,22 +770,27 @@ __global__ __launch_bounds__(kTraceBlock) void k_extend(TraceParams p, int q,
     uint32_t rays = 0;
     SceneView sv = scene_view(p.scene);
     auto begin = [&](uint32_t i, Trav &s) {
-        trav_begin_scene(s, v3{qo[i], qo[cap + i], qo[2 * cap + i]},
-                         v3{qd[i], qd[cap + i], qd[2 * cap + i]});
-        if (kShadow)
-        {
-            const uint32_t path = p.paths.qpath[2][i];
-            if (p.paths.neeTarget[path] == SPG_MISS) s.anyHit = true;
-            else s.out.t = p.paths.neeDist[path];
-        }
+        bool any = p.scene.instCount > 0;
         if (kBatch)
         {
             const DevScene &S =
                 p.scenes[p.slotItem[p.paths.pathSlot[p.paths.qpath[q][i]]]];
             sv = scene_view(S);
-            return S.instCount > 0;
+            any = S.instCount > 0;
         }
-        return p.scene.instCount > 0;
+        trav_begin_scene(sv, s, v3{qo[i], qo[cap + i], qo[2 * cap + i]},
+                         v3{qd[i], qd[cap + i], qd[2 * cap + i]});
+        if (kShadow)
+        {
+            const uint32_t path = p.paths.qpath[2][i];
+            if (p.paths.neeTarget[path] == SPG_MISS) s.anyHit = true;
+            else
+            {
+                s.out.t = p.paths.neeDist[path];
+                s.tc = world_cull(s.out.t);
+            }
+        }
+        return any;
     };
     auto store = [&](uint32_t i, const Trav &s) {
         p.paths.ht[i] = s.out.t;
@@ -1695,12 +1701,13 @@ static uint32_t device_cus()
 
 // Waves a persistent launch keeps resident: CUs x resident one-wave blocks
 // per CU, capped at kMaxPersistWavesPerCU per CU (the spill buffer size).
-template <class K> static uint32_t persistent_grid(K kernel)
+template <class K>
+static uint32_t persistent_grid(K kernel, uint32_t cap = kMaxPersistWavesPerCU)
 {
     int blocks = 0;
     hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, kTraceBlock, 0);
     if (blocks < 1) blocks = 1;
-    if (blocks > (int)kMaxPersistWavesPerCU) blocks = kMaxPersistWavesPerCU;
+    if (blocks > (int)cap) blocks = (int)cap;
     return device_cus() * (uint32_t)blocks;
 }
 
@@ -1710,14 +1717,18 @@ size_t spill_ints()
            (size_t)(kStackDepth - kMinShortStack);
 }
 
-static uint32_t persist_blocks(uint32_t grid, uint64_t n, uint32_t chunk = kSceneChunk)
+static uint32_t persist_blocks(uint32_t grid, uint32_t n)
 {
-    uint64_t need = (n + chunk - 1) / chunk;
-    if (need < 1) need = 1;
-    return need < grid ? (uint32_t)need : grid;
+    return std::min(walk_waves(n), grid);
 }
 
 __global__ void k_set_u32(uint32_t *p, uint32_t v) { *p = v; }
+
+// The mesh walk is bound by its node and triangle fetches (random rays
+// share few of them): more resident waves evict each other's lines from the
+// CU's 32 KB L1.  2^21 rays on 500k triangles: 8 waves per CU 516 us, 10
+// 513, 12 530; 300k rays on 100k triangles 264, 247, 243.
+constexpr uint32_t kMeshWavesPerCU = 10;
 
 hipError_t launch_closest_mesh(hipStream_t s, const DevMesh *mesh,
                                const float *ox, const float *oy,
@@ -1727,15 +1738,15 @@ hipError_t launch_closest_mesh(hipStream_t s, const DevMesh *mesh,
                                unsigned long long *stats, const Persist &ps)
 {
     if (n == 0) return hipSuccess;
-    static uint32_t gCount = persistent_grid(k_closest_mesh<true>);
-    static uint32_t gPlain = persistent_grid(k_closest_mesh<false>);
+    static uint32_t gCount = persistent_grid(k_closest_mesh<true>, kMeshWavesPerCU);
+    static uint32_t gPlain = persistent_grid(k_closest_mesh<false>, kMeshWavesPerCU);
     hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, ps.counter, 0u);
     if (stats)
-        hipLaunchKernelGGL(k_closest_mesh<true>, dim3(persist_blocks(gCount, n, kMeshChunk)),
+        hipLaunchKernelGGL(k_closest_mesh<true>, dim3(persist_blocks(gCount, n)),
                            dim3(kTraceBlock), 0, s, *mesh, ox, oy, oz, dx, dy, dz,
                            n, prim, t, u, v, stats, ps.counter, ps.spill);
     else
-        hipLaunchKernelGGL(k_closest_mesh<false>, dim3(persist_blocks(gPlain, n, kMeshChunk)),
+        hipLaunchKernelGGL(k_closest_mesh<false>, dim3(persist_blocks(gPlain, n)),
                            dim3(kTraceBlock), 0, s, *mesh, ox, oy, oz, dx, dy, dz,
                            n, prim, t, u, v, stats, ps.counter, ps.spill);
     return hipGetLastError();
@@ -1772,11 +1783,12 @@ hipError_t launch_closest_mesh_noalloc(hipStream_t s, const DevMesh *mesh,
                                        void *scratchPtr)
 {
     if (n == 0) return hipSuccess;
-    static uint32_t g = std::min(persistent_grid(k_closest_mesh<false>), kNoAllocWaves);
+    static uint32_t g =
+        std::min(persistent_grid(k_closest_mesh<false>, kMeshWavesPerCU), kNoAllocWaves);
     uint32_t *counter = (uint32_t *)scratchPtr;
     int *spill = (int *)((char *)scratchPtr + 256);
     hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s, counter, 0u);
-    hipLaunchKernelGGL(k_closest_mesh<false>, dim3(persist_blocks(g, n, kMeshChunk)),
+    hipLaunchKernelGGL(k_closest_mesh<false>, dim3(persist_blocks(g, n)),
                        dim3(kTraceBlock), 0, s, *mesh, ox, oy, oz, dx, dy, dz, n, prim,
                        t, u, v, nullptr, counter, spill);
     return hipGetLastError();

@@ -1,22 +1,31 @@
 // Closest-hit traversal as a per-lane step machine, run by persistent waves
 // that refill idle lanes with new rays.
 //
-// One loop iteration of a wave = one step per active lane, and every step
-// is one 64-byte fetch plus the arithmetic on it: a four-wide node visit
-// (decode and slab-test its quantized child boxes, order the hits by entry
-// distance), one triangle of the lane's current leaf, entering an
-// instance (its inverse transform and BVH) or leaving one after a hit (its
-// model transform, for the world-space t).  All lanes issue their fetch
-// together at the top of the step, so a wave whose lanes hold different
-// kinds of work waits for one memory round trip per iteration, not one per
-// kind.  A hit leaf child becomes the lane's leaf range (the nearest child
-// first, farther ones wait on the stack like inner nodes).  A lane whose
-// ray finishes takes the next ray from its wave's chunk of the ray list, so
-// the wave's SIMD lanes stay busy instead of idling behind the wave's longest
-// ray.  The two levels of a scene -- instance hierarchy (TLAS) and mesh
-// hierarchy (BLAS) -- are walked in the same loop: entering an instance
-// transforms the ray into mesh space (sp_RayIntersectScene,
-// src/sp_scene.cpp:263-276) and the mesh walk continues on the same stack.
+// A lane's next step is one of four kinds, each one 64-byte fetch plus the
+// arithmetic on it: a four-wide node visit (decode and slab-test its
+// quantized child boxes, order the hits by entry distance), one triangle of
+// the lane's current leaf, entering an instance (its inverse transform and
+// BVH) or leaving one after a hit (its model transform, for the world-space
+// t).  The walk is bound by vector instruction issue, and a wave pays for a
+// kind's instructions whether one of its lanes or all 64 are of that kind:
+// with every kind run in every iteration the 4M-triangle box scene took 253
+// instructions per ray and wave at 22% of the lanes busy.  So an iteration
+// runs ONE kind, the one that most lanes wait for (persistent_walk), and
+// the other lanes keep their state; what a lane does, and in which order,
+// does not depend on it.  A hit leaf child becomes the lane's leaf range
+// (the nearest child first, farther ones wait on the stack like inner
+// nodes).  A lane whose ray finishes takes the next ray from its wave's
+// chunk of the ray list, so the wave's SIMD lanes stay busy instead of
+// idling behind the wave's longest ray.  The two levels of a scene --
+// instance hierarchy (TLAS) and mesh hierarchy (BLAS) -- are walked in the
+// same loop: entering an instance transforms the ray into mesh space
+// (sp_RayIntersectScene, src/sp_scene.cpp:263-276) and the mesh walk
+// continues on the same stack.
+//
+// Measured against all kinds per iteration, per pass: 4M-triangle box scene
+// at 512x512 2397 -> 1757 us, 2.5M-triangle room at 1080p 5443 -> 4415,
+// eight-lamp scene with shadow rays 3979 -> 2784, 256x256 frame 361 -> 200,
+// 64x64 tile 110 -> 74; mesh rays: 2^21 on 500k triangles 664 -> 516.
 //
 // Stack: the top entries of each lane live in LDS (4 or 8 KB per wave);
 // deeper entries spill to a global array (rare: the builder bounds
@@ -28,26 +37,30 @@
 
 namespace spg {
 
-// Rays a wave takes from the shared counter with one atomic: the scene walk
-// of path-tracing rays is fastest at 64 (128: same, 256: -8% on the 4M-
-// triangle box scene), the single-mesh walk of incoherent rays at 128
-// (+23% over 64 on the 1M-triangle soup: with 64, the 65,536 same-address
-// atomics of a 2^22-ray launch serialize in L2; 256: -2% against 128).
-constexpr uint32_t kSceneChunk = 64, kMeshChunk = 128;
+// Rays a wave takes from the shared counter with one atomic, at most (a
+// short ray list is divided evenly among the waves): same-address atomics
+// serialize in L2, so 64 costs the mesh walk 44% at 2^21 rays (744 us
+// against 516), and the scene walk 1-3% (box 1771 -> 1757 us, eight lamps
+// 2861 -> 2784, room 4386 -> 4415).
+constexpr uint32_t kSceneChunk = 128, kMeshChunk = 128;
 // A wave refills its idle lanes once kRefill of them wait (or all do): each
 // refill stalls the wave on the new rays' loads and setup, so refilling one
 // lane per iteration adds a memory round trip to nearly every step, while
-// waiting for all 64 leaves the wave running its longest ray alone.  The
-// top kShort entries of each lane's stack live in LDS (kShort * 256 bytes
-// per wave), deeper ones spill to global memory.  Measured with four-wide
-// nodes: the scene walk (TLAS + BLAS, path-tracing rays of the 4M-triangle
-// box scene) is fastest at 40 / 16 (48: -4%, 56: -11%; 24 or 32 LDS
-// entries: -1%); the single-mesh walk of random rays (the 1M-triangle soup,
-// deeper stacks, longer rays) at 56 / 32 (+4% and +10% over 48 / 16).
-constexpr uint32_t kSceneRefill = 40, kMeshRefill = 56;
+// waiting for all 64 leaves the wave running its longest ray alone.  Scene
+// walk: 40 instead of 32 costs 2-3% (box 1820 against 1771 us, room 4532
+// against 4386); mesh walk: 48 instead of 32 costs 2% (527 against 516 us).
+constexpr uint32_t kSceneRefill = 32, kMeshRefill = 32;
+// The top kShort entries of each lane's stack live in LDS (kShort * 256
+// bytes per wave), deeper ones spill to global memory: 40 for the scene walk
+// costs the room 4% (4539 us against 4359), 80 for the mesh walk gains
+// nothing over 32.
 constexpr int kSceneShortStack = 16, kMeshShortStack = 32;
-constexpr int kMinShortStack = 16;  // sizes the spill area
-constexpr int32_t kNoRef = kEmptyChild;
+constexpr int kMinShortStack = 8;  // sizes the spill area
+// The weights of the step kinds when a wave chooses the kind to run: a lane
+// that waits for a rare kind costs as much as one that waits for a node, but
+// the node step is the longest (about 150 instructions against 60 to 90),
+// and a rare kind that waits until it has the most lanes waits for long.
+constexpr int kNodeWeight = 1, kTriangleWeight = 2, kEnterWeight = 3, kFinishWeight = 4;
 
 // Node, triangle and stack-spill arrays are reached through pointers read
 // from memory (mesh and scene tables), so the compiler cannot prove them
@@ -66,7 +79,18 @@ __device__ __forceinline__ float4 ld_g4(const float4 *p)
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
-__device__ __forceinline__ bool d_is_leaf(int32_t r) { return r < 0; }
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(1))) f2v gf2v;
+typedef const __attribute__((address_space(1))) float gf1;
+
+__device__ __forceinline__ float2 ld_g2(const float4 *p)
+{
+    f2v v = *(gf2v *)p;
+    return make_float2(v.x, v.y);
+}
+
+__device__ __forceinline__ float ld_g1(const float4 *p) { return *(gf1 *)p; }
+
 __device__ __forceinline__ uint32_t d_leaf_first(int32_t r)
 {
     return ((uint32_t)~r) >> 3;
@@ -106,10 +130,30 @@ struct LaneStack
         if (i < kShort) lds[i * 64 + lane] = v;
         else spill[(size_t)(i - kShort) * stride + gl] = v;
     }
+    // Entries i, i + 1, i + 2; only the first n are live (the others are
+    // above the stack top, so what they hold does not matter and the LDS
+    // case writes all three without a branch).
+    __device__ __forceinline__ void write3(int i, int n, int v0, int v1, int v2)
+    {
+        if (__ballot(i + 3 > kShort) == 0ull)
+        {
+            lint *at = lds + i * 64 + lane;
+            at[0] = v0;
+            at[64] = v1;
+            at[128] = v2;
+        }
+        else
+        {
+            if (n > 0) write(i, v0);
+            if (n > 1) write(i + 1, v1);
+            if (n > 2) write(i + 2, v2);
+        }
+    }
     __device__ __forceinline__ int read(int i)
     {
         int v;
-        if (i < kShort) v = lds[i * 64 + lane];
+        if (__ballot(i >= kShort) == 0ull) v = lds[i * 64 + lane];
+        else if (i < kShort) v = lds[i * 64 + lane];
         else v = spill[(size_t)(i - kShort) * stride + gl];
         return v;
     }
@@ -130,26 +174,31 @@ __device__ __forceinline__ SceneView scene_view(const DevScene &S)
 
 struct Trav
 {
-    v3 o, d, inv;              // world ray
-    v3 lo, ld, linv;           // ray in the current mesh's space
-    const float4 *bnodes;      // the mesh's records: nodes, then triangles
-    float lim;                 // bound on the mesh-space t from the world best
+    v3 o, inv;                 // ray of the current level (world, or mesh space)
+    v3 ld;                     // mesh-space direction
+    v3 wo, wd, winv;           // world ray
+    const float4 *nodes;       // records of the current level (a mesh's: nodes,
+                               // then triangles)
+    float tc;                  // t cull of the current level: the best hit's
+                               // bound with the slack
     Hit h;                     // best hit in the current mesh
     SceneHit out;              // best hit in the scene
-    int node, sp, spBase, level;
-    uint32_t inst;
-    uint32_t triNext, triEnd;  // pending triangles of the current leaf
-    uint32_t mode;             // the next step's work (kMode*)
-    bool mmW, mmL;             // world / mesh-space ray is finite
+    int32_t cur;               // the lane's next step: a node (>= 0), a leaf
+                               // (< 0: triangles in a mesh, an instance in
+                               // the instance hierarchy) or kFinishStep / kNoStep
+    int sp, spBase;            // stack entries; where the mesh's begin (-1:
+                               // in the instance hierarchy)
+    uint32_t inst;             // the instance walked
+    bool mm, mmW;              // the current level's / the world ray is finite
     bool anyHit;               // occlusion query: stop at the first instance
                                // hit with a positive world t
 };
 
-// Kinds of step.
-constexpr uint32_t kModeNode = 0;    // visit node `node` of the current level
-constexpr uint32_t kModeTri = 1;     // test triangle triNext of the leaf range
-constexpr uint32_t kModeEnter = 2;   // enter instance `inst`
-constexpr uint32_t kModeFinish = 3;  // leave instance `inst` with its hit
+// Values of Trav::cur that are not references (node indices stay below
+// 2^28).
+constexpr int32_t kFinishStep = 0x7FFFFFFD;  // leave the instance with its hit
+constexpr int32_t kNoStep = 0x7FFFFFFC;      // no walk: idle or complete
+constexpr uint32_t kFirstStepCode = 0x7FFFFFFC;
 
 // Moller-Trumbore on one fetched triangle record (a.xyz, e1.x) (e1.yz,
 // e2.xy) (e2.z, prim, n.xy) (n.z, ...) with n = cross(e1, e2) stored
@@ -173,66 +222,150 @@ __device__ __forceinline__ m34 rows3(float4 a, float4 b, float4 c)
     return m34{{{a.x, a.y, a.z, a.w}, {b.x, b.y, b.z, b.w}, {c.x, c.y, c.z, c.w}}};
 }
 
-// One step of an active lane (an inactive lane's state is left as it is).
-// Returns true when the ray's walk is complete.  kTwoLevel = false walks a
-// single mesh (level stays 1, spBase 0; only node and triangle steps).
-//
-// Loads and arithmetic sit in branches; the lane state is written through
-// selects after them, and the step runs on every lane with `active` in its
-// predicates.  Written inside divergent branches, every state value needs a
-// second register at each join and the compiler copies the whole state
-// around every branch of the step.
-template <bool kCount, bool kTwoLevel, int kShort>
-__device__ __forceinline__ bool trav_step(const SceneView &sv, Trav &s,
-                                         LaneStack<kShort> &st, Counts &cnt,
-                                         bool active)
+// The t cull in the instance hierarchy.
+__device__ __forceinline__ float world_cull(float t)
 {
-    const uint32_t mode = s.mode;
-    const bool blas = !kTwoLevel || s.level != 0;
+    return t > 0.0f ? t * kCullSlack : INFINITY;
+}
 
-    // (1) the step's 64-byte fetch: a node or triangle record of the mesh,
-    // a TLAS node, instance bytes 48..111 (enter) or 0..63 (leave)
-    const float4 *src;
-    if (!kTwoLevel || mode <= kModeTri)
-        src = (blas ? s.bnodes : sv.tlasNodes) +
-              4 * (mode == kModeTri ? (int)s.triNext : s.node);
-    else
-        src = reinterpret_cast<const float4 *>(sv.inst + s.inst) +
-              (mode == kModeEnter ? 3 : 0);
-    float4 A, B, C, D;  // read only by active lanes
-    if (active)
+// What the lanes of a step (`act`) do after it: a lane with `need` has
+// nothing to descend into; it leaves a finished mesh walk (by a step of its
+// own when it found a hit, at once without one), then pops; with an empty
+// stack its walk is complete.  Any other lane goes on with `next`.
+//
+// The fetch and its arithmetic sit in branches on `act`; the state is
+// written through selects after them, in straight code that every lane runs:
+// written inside nested divergent branches, each value would need a second
+// register at every join and be copied into it on the way.
+template <bool kTwoLevel, int kShort>
+__device__ __forceinline__ void trav_advance(const SceneView &sv, Trav &s,
+                                             LaneStack<kShort> &st, bool act, bool need,
+                                             int32_t next)
+{
+    need = need && act;
+    bool fin = false;
+    if (kTwoLevel)
     {
-        A = ld_g4(src);
-        B = ld_g4(src + 1);
-        C = ld_g4(src + 2);
-        D = ld_g4(src + 3);
+        const bool end = need && s.sp <= s.spBase;
+        const bool hit = s.h.prim != SPG_MISS;
+        fin = end && hit;
+        const bool leave = end && !hit;
+        const float wt = world_cull(s.out.t);
+        s.o = v3{leave ? s.wo.x : s.o.x, leave ? s.wo.y : s.o.y, leave ? s.wo.z : s.o.z};
+        s.inv = v3{leave ? s.winv.x : s.inv.x, leave ? s.winv.y : s.inv.y,
+                   leave ? s.winv.z : s.inv.z};
+        s.mm = leave ? s.mmW : s.mm;
+        s.nodes = leave ? sv.tlasNodes : s.nodes;
+        s.tc = leave ? wt : s.tc;
+        s.spBase = leave ? -1 : s.spBase;
     }
+    const bool pop = need && !fin && s.sp != 0;
+    int v = 0;
+    if (pop) v = st.read(s.sp - 1);
+    s.sp -= pop ? 1 : 0;
+    const int32_t popped = fin ? kFinishStep : pop ? v : kNoStep;
+    s.cur = !act ? s.cur : need ? popped : next;
+}
 
-    // (2) the work on it
-    const bool isTri = active && mode == kModeTri;
-    const bool isNode = active && mode == kModeNode;
-    const bool isEnter = kTwoLevel && active && mode == kModeEnter;
-    const bool isFin = kTwoLevel && active && mode == kModeFinish;
-    Hit c{0.0f, 0.0f, 0.0f, 0u};
-    bool take = false;
-    int32_t next = kNoRef;
-    // pending children of a node visit, stored at sp, sp + 1, sp + 2
-    int32_t push0 = kNoRef, push1 = kNoRef, push2 = kNoRef;
-    int npush = 0;
-    if (isTri)
-        take = triangle_candidate(A, B, C, D, s.lo, s.ld, s.h, c);
-    else if (isNode)
+// The four bytes of a word as halves of value q 2^-24 (subnormal halves):
+// bytes 0, 1 and bytes 2, 3.
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ h2 halves_lo(uint32_t w)
+{
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, w, 0x0C010C00u));
+}
+__device__ __forceinline__ h2 halves_hi(uint32_t w)
+{
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, w, 0x0C030C02u));
+}
+
+// v_min_f64 / v_max_f64 of two numbers (fmin and fmax would first quiet
+// operands that cannot be NaN here).
+__device__ __forceinline__ double min_f64(double a, double b)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double max_f64(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// The sort key of a missed or absent child: above every entry distance.
+constexpr uint32_t kMissKey = 0x7FE00000u;
+
+// A hit child's key: the entry distance's bits with the sign cleared
+// (-0 = +0) and the two low bits replaced by the child slot, so keys are
+// distinct and near-ties go to the lower slot; a missed or absent child gets
+// the largest key.
+__device__ __forceinline__ uint32_t child_key(int k, bool hit, float e)
+{
+    return hit ? ((__float_as_uint(e) & 0x7FFFFFFCu) | (uint32_t)k) : kMissKey;
+}
+
+// The child keys of a node for a ray that step_node's fast form does not
+// cover (rare; the node is read again so that its words stay out of the
+// registers of the common path).
+__device__ __forceinline__ void slow_keys(const float4 *src, bool mm, v3 o, v3 inv, float tc,
+                                          uint32_t (&key)[4])
+{
+    asm volatile("" : "+v"(src));
+    const float4 A = ld_g4(src), B = ld_g4(src + 1), C = ld_g4(src + 2);
+    const float2 D = ld_g2(src + 3);
+    const uint32_t eb = __float_as_uint(A.w);
+    const float sx = __uint_as_float((eb & 0xFFu) << 23);
+    const float sy = __uint_as_float(((eb >> 8) & 0xFFu) << 23);
+    const float sz = __uint_as_float(((eb >> 16) & 0xFFu) << 23);
+    const uint32_t q[6] = {__float_as_uint(C.x), __float_as_uint(C.y), __float_as_uint(C.z),
+                           __float_as_uint(C.w), __float_as_uint(D.x), __float_as_uint(D.y)};
+    const int32_t ref[4] = {__float_as_int(B.x), __float_as_int(B.y), __float_as_int(B.z),
+                            __float_as_int(B.w)};
+    const v3 a{sx * inv.x, sy * inv.y, sz * inv.z};
+    const v3 b{(A.x - o.x) * inv.x, (A.y - o.y) * inv.y, (A.z - o.z) * inv.z};
+    const bool fold = mm && finite3(a) && finite3(b);
+    const bool px = inv.x > 0.0f, py = inv.y > 0.0f, pz = inv.z > 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
     {
-        v3 o = blas ? s.lo : s.o;
-        v3 inv = blas ? s.linv : s.inv;
-        float tc;
-        if (blas)
-        {
-            tc = s.h.t * kCullSlack;
-            tc = tc < s.lim ? tc : s.lim;
-        }
+        auto dq = [&](int f, float sc, float p) {
+            return fmaf((float)((q[f] >> (8 * k)) & 0xFFu), sc, p);
+        };
+        float e;
+        bool h;
+        if (fold)
+            // only a 2^24 overflows: the same distances, unscaled
+            h = slab_hit_t(dq(px ? 0 : 3, a.x, b.x), dq(py ? 1 : 4, a.y, b.y),
+                           dq(pz ? 2 : 5, a.z, b.z), dq(px ? 3 : 0, a.x, b.x),
+                           dq(py ? 4 : 1, a.y, b.y), dq(pz ? 5 : 2, a.z, b.z), &e);
         else
-            tc = s.out.t > 0.0f ? s.out.t * kCullSlack : INFINITY;
+            // a non-finite origin, inverse direction or per-axis factor (an
+            // axis-parallel ray, or s inv overflowing): the reference's
+            // compare-and-select form on the decoded box
+            h = slab_hit(dq(0, sx, A.x), dq(1, sy, A.y), dq(2, sz, A.z), dq(3, sx, A.x),
+                         dq(4, sy, A.y), dq(5, sz, A.z), o, inv, &e);
+        key[k] = child_key(k, h && e <= tc && ref[k] != kEmptyChild, e);
+    }
+}
+
+// One node visit: decode and slab-test the children, the nearest hit one is
+// the next step and the others go to the stack.
+template <bool kCount, bool kTwoLevel, int kShort>
+__device__ __forceinline__ void step_node(const SceneView &sv, Trav &s,
+                                          LaneStack<kShort> &st, Counts &cnt, bool act)
+{
+    int npush = 0;
+    int32_t push0 = 0, push1 = 0, push2 = 0, next = kNoStep;
+    bool none = false;
+    if (act)
+    {
+        const float4 *src = s.nodes + 4 * (size_t)(uint32_t)s.cur;
+        const float4 A = ld_g4(src), B = ld_g4(src + 1), C = ld_g4(src + 2);
+        const float2 D = ld_g2(src + 3);
+        const v3 o = s.o, inv = s.inv;
+        const float tc = s.tc;
         // A: origin p and scale exponents; B: child references; C, D: the
         // child boxes, one field of all four children per 32-bit word.  A
         // coordinate decodes to p + q * s: q * s is exact (8-bit integer
@@ -244,249 +377,260 @@ __device__ __forceinline__ bool trav_step(const SceneView &sv, Trav &s,
         const uint32_t q0 = __float_as_uint(C.x), q1 = __float_as_uint(C.y),
                        q2 = __float_as_uint(C.z), q3 = __float_as_uint(C.w),
                        q4 = __float_as_uint(D.x), q5 = __float_as_uint(D.y);
-        int32_t ref[4] = {__float_as_int(B.x), __float_as_int(B.y),
-                          __float_as_int(B.z), __float_as_int(B.w)};
-        auto dq = [](uint32_t w, int k, float sc, float p) {
-            return fmaf((float)((w >> (8 * k)) & 0xFFu), sc, p);
-        };
-        // a hit child's key: the entry distance's bits with the sign
-        // cleared (-0 = +0) and the two low bits replaced by the child slot,
-        // so keys are distinct and near-ties go to the lower slot; a missed
-        // or absent child gets the largest key
-        auto keyOf = [&](int k, bool h, float e) {
-            return (h & (e <= tc) & (ref[k] != kEmptyChild))
-                       ? ((__float_as_uint(e) & 0x7FFFFFFCu) | (uint32_t)k)
-                       : 0xFFFFFFFFu;
-        };
+        int32_t ref[4] = {__float_as_int(B.x), __float_as_int(B.y), __float_as_int(B.z),
+                          __float_as_int(B.w)};
         uint32_t key[4];
         // a plane at p + q s (q the 8-bit field) is crossed at
         // t = (p + q s - o) inv = q (s inv) + (p - o) inv: per node and axis
         // a = s inv (exact: s is a power of two) and b = (p - o) inv, then
-        // one FMA per plane
+        // one FMA per plane.  The byte q is spread into a half whose bits read
+        // as the subnormal q 2^-24, so the multiply-add that widens a half
+        // operand takes it without a conversion: (q 2^-24) (a 2^24) + b, the
+        // same product and rounding.
         const float ax = sx * inv.x, ay = sy * inv.y, az = sz * inv.z;
         const float bx = (A.x - o.x) * inv.x, by = (A.y - o.y) * inv.y,
                     bz = (A.z - o.z) * inv.z;
-        const bool fold = (blas ? s.mmL : s.mmW) && finite3(v3{ax, ay, az}) &&
-                          finite3(v3{bx, by, bz});
+        const float cx24 = ax * 16777216.0f, cy24 = ay * 16777216.0f, cz24 = az * 16777216.0f;
+        // finite factors (with a finite ray none can be NaN: |s|, |p - o| and
+        // |inv| are numbers, so a product is finite or infinite)
+        const float big =
+            fmaxf(fmaxf(fmaxf(fabsf(cx24), fabsf(cy24)), fmaxf(fabsf(cz24), fabsf(bx))),
+                  fmaxf(fabsf(by), fabsf(bz)));
+        const bool fast = s.mm && big < INFINITY;
+        // per axis the near plane is the lo field where inv > 0 (a
+        // positive a makes t increase with q) and the hi field where
+        // inv < 0, so choosing the fields once per node orders each
+        // axis's two distances
+        const bool px = inv.x > 0.0f, py = inv.y > 0.0f, pz = inv.z > 0.0f;
+        const uint32_t nx = px ? q0 : q3, fx = px ? q3 : q0;
+        const uint32_t ny = py ? q1 : q4, fy = py ? q4 : q1;
+        const uint32_t nz = pz ? q2 : q5, fz = pz ? q5 : q2;
         {
-            // per axis the near plane is the lo field where inv > 0 (a
-            // positive a makes t increase with q) and the hi field where
-            // inv < 0, so choosing the fields once per node orders each
-            // axis's two distances
-            const bool px = inv.x > 0.0f, py = inv.y > 0.0f, pz = inv.z > 0.0f;
-            const uint32_t nx = px ? q0 : q3, fx = px ? q3 : q0;
-            const uint32_t ny = py ? q1 : q4, fy = py ? q4 : q1;
-            const uint32_t nz = pz ? q2 : q5, fz = pz ? q5 : q2;
+            const h2 nx0 = halves_lo(nx), nx1 = halves_hi(nx), fx0 = halves_lo(fx),
+                     fx1 = halves_hi(fx), ny0 = halves_lo(ny), ny1 = halves_hi(ny),
+                     fy0 = halves_lo(fy), fy1 = halves_hi(fy), nz0 = halves_lo(nz),
+                     nz1 = halves_hi(nz), fz0 = halves_lo(fz), fz1 = halves_hi(fz);
 #pragma unroll
             for (int k = 0; k < 4; ++k)
             {
+                const int i = k & 1;
+                auto pl = [&](h2 l, h2 h, float c, float b) {
+                    return fmaf((float)(k < 2 ? l[i] : h[i]), c, b);
+                };
                 float e;
-                bool h = slab_hit_t(dq(nx, k, ax, bx), dq(ny, k, ay, by), dq(nz, k, az, bz),
-                                    dq(fx, k, ax, bx), dq(fy, k, ay, by), dq(fz, k, az, bz),
-                                    &e);
-                key[k] = keyOf(k, h, e);
+                bool h = slab_hit_t(pl(nx0, nx1, cx24, bx), pl(ny0, ny1, cy24, by),
+                                    pl(nz0, nz1, cz24, bz), pl(fx0, fx1, cx24, bx),
+                                    pl(fy0, fy1, cy24, by), pl(fz0, fz1, cz24, bz), &e);
+                key[k] = child_key(k, h & (e <= tc) & (ref[k] != kEmptyChild), e);
             }
         }
-        if (!fold)
-        {
-            // a non-finite origin, inverse direction or per-axis factor (an
-            // axis-parallel ray, or s inv overflowing): the reference's
-            // compare-and-select form on the decoded box
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-            {
-                float e;
-                bool h = slab_hit(dq(q0, k, sx, A.x), dq(q1, k, sy, A.y),
-                                  dq(q2, k, sz, A.z), dq(q3, k, sx, A.x),
-                                  dq(q4, k, sy, A.y), dq(q5, k, sz, A.z), o, inv, &e);
-                key[k] = keyOf(k, h, e);
-            }
-        }
+        if (!fast) slow_keys(src, s.mm, o, inv, tc, key);
         if (kCount)
         {
             uint32_t present = 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) present += ref[k] != kEmptyChild ? 1u : 0u;
-            if (blas) cnt.box += present;
+            if (!kTwoLevel || s.spBase >= 0) cnt.box += present;
             else cnt.tlasBox += present;
         }
-        // sort (key, reference) pairs by key: five compare-exchanges
+        // sort (key, reference) pairs by key: five compare-exchanges.  A pair is
+        // one 64-bit word, key above reference; as a double it is positive and
+        // finite (keys stay below 0x7FF00000), so the double minimum and maximum
+        // order the words as integers, subnormals included, in two operations
+        // per exchange instead of a compare and four selects.
+        double pr[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            pr[k] = __longlong_as_double(
+                (long long)(((uint64_t)key[k] << 32) | (uint32_t)ref[k]));
         auto cx = [&](int a, int b) {
-            const bool sw = key[b] < key[a];
-            const uint32_t lo = sw ? key[b] : key[a], hi = sw ? key[a] : key[b];
-            const int32_t ra = sw ? ref[b] : ref[a], rb = sw ? ref[a] : ref[b];
-            key[a] = lo;
-            key[b] = hi;
-            ref[a] = ra;
-            ref[b] = rb;
+            const double lo = min_f64(pr[a], pr[b]), hi = max_f64(pr[a], pr[b]);
+            pr[a] = lo;
+            pr[b] = hi;
         };
         cx(0, 1);
         cx(2, 3);
         cx(0, 2);
         cx(1, 3);
         cx(1, 2);
+        auto miss = [&](int k) { return __double2hiint(pr[k]) == (int)kMissKey; };
+        auto refOf = [&](int k) { return (int32_t)__double2loint(pr[k]); };
         // the nearest is next; the others wait on the stack, the nearest
         // of them on top: slot 3 at sp, slot 2 above it, slot 1 on top
-        const bool v1 = key[1] != 0xFFFFFFFFu, v2 = key[2] != 0xFFFFFFFFu,
-                   v3 = key[3] != 0xFFFFFFFFu;
-        next = key[0] != 0xFFFFFFFFu ? ref[0] : kNoRef;
-        push0 = v3 ? ref[3] : v2 ? ref[2] : ref[1];
-        push1 = v3 ? ref[2] : ref[1];
-        push2 = ref[1];
+        const bool v1 = !miss(1), v2 = !miss(2), v3 = !miss(3);
         npush = (v1 ? 1 : 0) + (v2 ? 1 : 0) + (v3 ? 1 : 0);
+        push0 = v3 ? refOf(3) : v2 ? refOf(2) : refOf(1);
+        push1 = v3 ? refOf(2) : refOf(1);
+        push2 = refOf(1);
+        next = refOf(0);
+        none = miss(0);
+    }
+    if (__ballot(npush != 0) != 0ull) st.write3(s.sp, npush, push0, push1, push2);
+    s.sp += npush;
+    trav_advance<kTwoLevel>(sv, s, st, act, none, next);
+}
+
+// One triangle of the lane's leaf; after the last one the lane pops.
+template <bool kCount, bool kTwoLevel, int kShort>
+__device__ __forceinline__ void step_triangle(const SceneView &sv, Trav &s,
+                                              LaneStack<kShort> &st, Counts &cnt, bool act)
+{
+    Hit c{0.0f, 0.0f, 0.0f, 0u};
+    bool take = false;
+    if (act)
+    {
+        const float4 *src = s.nodes + 4 * (size_t)d_leaf_first(s.cur);
+        const float4 A = ld_g4(src), B = ld_g4(src + 1), C = ld_g4(src + 2);
+        const float4 D = make_float4(ld_g1(src + 3), 0.0f, 0.0f, 0.0f);
+        take = triangle_candidate(A, B, C, D, s.o, s.ld, s.h, c);
     }
     s.h.t = take ? c.t : s.h.t;
     s.h.u = take ? c.u : s.h.u;
     s.h.v = take ? c.v : s.h.v;
     s.h.prim = take ? c.prim : s.h.prim;
-    s.triNext += isTri ? 1u : 0u;
-    if (npush > 0) st.write(s.sp, push0);
-    if (npush > 1) st.write(s.sp + 1, push1);
-    if (npush > 2) st.write(s.sp + 2, push2);
-    s.sp += npush;
-    const bool busy = isTri && s.triNext < s.triEnd;
-
-    bool stop = false;  // an occlusion query found a hit
-    if (kTwoLevel)
-    {
-        // entering: o' = M^-1 o, d' = norm(M^-1 d) (src/sp_scene.cpp:272-276);
-        // the mesh walk starts at its root above the current stack
-        v3 nlo{0.0f, 0.0f, 0.0f}, nld{0.0f, 0.0f, 0.0f}, nlinv{0.0f, 0.0f, 0.0f};
-        float nlim = 0.0f;
-        bool nmm = false;
-        const float4 *nb = nullptr;
-        if (isEnter)
-        {
-            const m34 I = rows3(A, B, C);
-            nlo = xform_point(I, s.o);
-            nld = normalize(xform_vector(I, s.d));
-            nlinv = inverse(nld);
-            nmm = finite3(nlo) && finite3(nlinv);
-            nlim = s.out.t > 0.0f ? s.out.t * D.x * kCullSlack : INFINITY;
-            nb = reinterpret_cast<const float4 *>(
-                ((uint64_t)__float_as_uint(D.w) << 32) | __float_as_uint(D.z));
-        }
-        s.lo = v3{isEnter ? nlo.x : s.lo.x, isEnter ? nlo.y : s.lo.y,
-                  isEnter ? nlo.z : s.lo.z};
-        s.ld = v3{isEnter ? nld.x : s.ld.x, isEnter ? nld.y : s.ld.y,
-                  isEnter ? nld.z : s.ld.z};
-        s.linv = v3{isEnter ? nlinv.x : s.linv.x, isEnter ? nlinv.y : s.linv.y,
-                    isEnter ? nlinv.z : s.linv.z};
-        s.lim = isEnter ? nlim : s.lim;
-        s.mmL = isEnter ? nmm : s.mmL;
-        s.bnodes = isEnter ? nb : s.bnodes;
-        s.h.t = isEnter ? INFINITY : s.h.t;
-        s.h.prim = isEnter ? SPG_MISS : s.h.prim;
-        s.spBase = isEnter ? s.sp : s.spBase;
-        if (kCount) cnt.mesh += isEnter ? 1u : 0u;
-
-        // leaving with a hit: world t = dot(M (o' + t' d') - o, d), the
-        // closest world hit wins (src/sp_scene.cpp:296-322), equal t goes to
-        // the lower instance index
-        bool better = false;
-        float tw = 0.0f;
-        if (isFin)
-        {
-            v3 lh = s.lo + s.ld * s.h.t;
-            v3 wh = xform_point(rows3(A, B, C), lh);
-            tw = dot(wh - s.o, s.d);
-            // an occlusion query takes the first instance hit at a positive
-            // world t (what k_resolve_shadow counts as a blocker) and stops;
-            // a hit whose world t rounds to <= 0 neither stops nor blocks
-            better = s.anyHit ? tw > 0.0f
-                              : tw < s.out.t || s.out.t < 0.0f ||
-                                    (tw == s.out.t && s.inst < s.out.inst);
-        }
-        stop = s.anyHit & better;
-        s.out.t = better ? tw : s.out.t;
-        s.out.u = better ? s.h.u : s.out.u;
-        s.out.v = better ? s.h.v : s.out.v;
-        s.out.inst = better ? s.inst : s.out.inst;
-        s.out.prim = better ? s.h.prim : s.out.prim;
-        s.level = isEnter ? 1 : isFin ? 0 : s.level;
-    }
-
-    // (3) the next work.  Nothing to descend into: leave a finished mesh
-    // walk (at once without a hit, by a leave step with one), then pop.  A
-    // popped reference is never empty, so one pop gives the next step work.
-    bool needPop = (isNode && next == kNoRef) || (isTri && !busy) || isFin;
-    bool leaveStep = false;
-    if (kTwoLevel)
-    {
-        const bool leave = needPop && s.level != 0 && s.sp <= s.spBase;
-        leaveStep = leave && s.h.prim != SPG_MISS;
-        s.level = leave && !leaveStep ? 0 : s.level;
-        needPop = needPop && !leaveStep;
-    }
-    const bool done = (needPop && s.sp == 0) || stop;
-    const bool doPop = needPop && s.sp != 0;
-    int32_t popped = kNoRef;
-    if (doPop) popped = st.read(s.sp - 1);
-    s.sp -= doPop ? 1 : 0;
-    next = doPop ? popped : next;
-
-    const bool leaf = d_is_leaf(next);
-    const bool enter = kTwoLevel && leaf && s.level == 0;
-    const bool range = leaf && !enter;
-    const bool inner = !leaf && next != kNoRef;
-    const uint32_t first = d_leaf_first(next), count = d_leaf_count(next);
-    s.triNext = range ? first : s.triNext;
-    s.triEnd = range ? first + count : s.triEnd;
-    if (kCount) cnt.tri += range ? count : 0u;
-    s.inst = enter ? first : s.inst;
-    s.node = inner ? next : isEnter ? 0 : s.node;
-    s.mode = leaveStep ? kModeFinish
-             : enter   ? kModeEnter
-             : range   ? kModeTri
-             : (inner || isEnter) ? kModeNode
-             : busy    ? kModeTri
-                       : s.mode;
-    return done;
+    const float ts = c.t * kCullSlack;
+    s.tc = take && ts < s.tc ? ts : s.tc;
+    if (kCount) cnt.tri += act ? 1u : 0u;
+    // ~cur = first * 8 + (count - 1): the next triangle is first + 1,
+    // count - 1, which is ~cur + 7
+    trav_advance<kTwoLevel>(sv, s, st, act, d_leaf_count(s.cur) == 1u,
+                            (int32_t)((uint32_t)s.cur - 7u));
 }
 
-__device__ __forceinline__ void trav_begin_scene(Trav &s, v3 o, v3 d)
+// Entering instance (leaf): o' = M^-1 o, d' = norm(M^-1 d)
+// (src/sp_scene.cpp:272-276); the mesh walk starts at its root above the
+// current stack.
+template <bool kCount>
+__device__ __forceinline__ void step_enter(const SceneView &sv, Trav &s, Counts &cnt, bool act)
 {
-    s.o = o;
-    s.d = d;
-    s.inv = inverse(d);
-    s.mmW = finite3(o) && finite3(s.inv);
-    s.mmL = false;
+    if (act)
+    {
+        s.inst = d_leaf_first(s.cur);
+        const float4 *src = reinterpret_cast<const float4 *>(sv.inst + s.inst) + 3;
+        const float4 A = ld_g4(src), B = ld_g4(src + 1), C = ld_g4(src + 2), D = ld_g4(src + 3);
+        const m34 I = rows3(A, B, C);
+        s.o = xform_point(I, s.wo);
+        s.ld = normalize(xform_vector(I, s.wd));
+        s.inv = inverse(s.ld);
+        s.mm = finite3(s.o) && finite3(s.inv);
+        s.tc = s.out.t > 0.0f ? s.out.t * D.x * kCullSlack : INFINITY;
+        s.nodes = reinterpret_cast<const float4 *>(
+            ((uint64_t)__float_as_uint(D.w) << 32) | __float_as_uint(D.z));
+        s.h.t = INFINITY;
+        s.h.prim = SPG_MISS;
+        s.spBase = s.sp;
+        s.cur = 0;
+        if (kCount) cnt.mesh += 1u;
+    }
+}
+
+// Leaving an instance with a hit: world t = dot(M (o' + t' d') - o, d), the
+// closest world hit wins (src/sp_scene.cpp:296-322), equal t goes to the
+// lower instance index.
+template <int kShort>
+__device__ __forceinline__ void step_finish(const SceneView &sv, Trav &s,
+                                            LaneStack<kShort> &st, bool act)
+{
+    float tw = 0.0f;
+    if (act)
+    {
+        const float4 *src = reinterpret_cast<const float4 *>(sv.inst + s.inst);
+        const float4 A = ld_g4(src), B = ld_g4(src + 1), C = ld_g4(src + 2);
+        const v3 lh = s.o + s.ld * s.h.t;
+        const v3 wh = xform_point(rows3(A, B, C), lh);
+        tw = dot(wh - s.wo, s.wd);
+    }
+    // an occlusion query takes the first instance hit at a positive
+    // world t (what k_resolve_shadow counts as a blocker) and stops;
+    // a hit whose world t rounds to <= 0 neither stops nor blocks
+    const bool closer = tw < s.out.t || s.out.t < 0.0f ||
+                        (tw == s.out.t && s.inst < s.out.inst);
+    const bool better = act && (s.anyHit ? tw > 0.0f : closer);
+    s.out.t = better ? tw : s.out.t;
+    s.out.u = better ? s.h.u : s.out.u;
+    s.out.v = better ? s.h.v : s.out.v;
+    s.out.inst = better ? s.inst : s.out.inst;
+    s.out.prim = better ? s.h.prim : s.out.prim;
+    s.h.prim = act ? SPG_MISS : s.h.prim;
+    // an occlusion query that found a blocker is complete
+    trav_advance<true>(sv, s, st, act, !(s.anyHit && better), kNoStep);
+}
+
+__device__ __forceinline__ void trav_begin_scene(const SceneView &sv, Trav &s, v3 o, v3 d)
+{
+    s.o = s.wo = o;
+    s.wd = d;
+    s.inv = s.winv = inverse(d);
+    s.mm = s.mmW = finite3(o) && finite3(s.inv);
+    s.nodes = sv.tlasNodes;
+    s.tc = INFINITY;
     s.anyHit = false;
     s.out = SceneHit{-1.0f, 0.0f, 0.0f, SPG_MISS, SPG_MISS};
-    s.level = 0;
     s.sp = 0;
-    s.spBase = 0;
-    s.node = 0;
-    s.h = Hit{INFINITY, 0.0f, 0.0f, SPG_MISS};
-    s.triNext = s.triEnd = 0;
-    s.mode = kModeNode;
+    s.spBase = -1;
+    s.cur = 0;
 }
 
 __device__ __forceinline__ void trav_begin_mesh(const DevMesh &M, Trav &s, v3 o,
                                                 v3 d)
 {
-    s.lo = o;
+    s.o = o;
     s.ld = d;
-    s.linv = inverse(d);
-    s.mmL = finite3(o) && finite3(s.linv);
-    s.mmW = false;
-    s.anyHit = false;
-    s.bnodes = M.nodes;
-    s.lim = INFINITY;
+    s.inv = inverse(d);
+    s.mm = finite3(o) && finite3(s.inv);
+    s.nodes = M.nodes;
+    s.tc = INFINITY;
     s.h = Hit{INFINITY, 0.0f, 0.0f, SPG_MISS};
-    s.level = 1;
     s.sp = 0;
-    s.spBase = 0;
-    s.node = 0;
-    s.triNext = s.triEnd = 0;
-    s.mode = kModeNode;
+    s.cur = 0;
 }
 
-// Persistent driver: every wave walks rays [0, n) taken in chunks of
-// kChunk from *counter (zero on entry), refilling its idle lanes once
-// `refill` (1..64, wave-uniform) of them wait.  begin(ray, s) starts a ray
-// and returns false if it needs no walk (it is then stored at once);
-// store(ray, s) writes the result.  Must be called by every lane of a
+// The rays of a persistent launch in chunks, handed to its waves: chunk j
+// holds rays [j * chunk, (j + 1) * chunk).  A wave's first chunk is the one
+// at its own position, the further ones come from the counter (zero on
+// entry), so a launch whose rays fit its waves makes no atomic at all and in
+// the others no wave starts by waiting for one (same-address atomics take
+// 11 ns each: 56 us for 5120 waves that start together).
+struct WorkSource
+{
+    uint32_t *counter;
+    uint32_t n, waves, chunk, chunks;
+    bool first;
+    __device__ __forceinline__ WorkSource(uint32_t *c, uint32_t rays, uint32_t w,
+                                          uint32_t maxChunk)
+        : counter(c), n(rays), waves(w), first(true)
+    {
+        const uint32_t last = n ? n - 1u : 0u;  // (n + waves - 1 could wrap)
+        chunk = min(last / waves + 1u, maxChunk);
+        chunks = n ? last / chunk + 1u : 0u;
+    }
+    // The wave's next chunk as rays [lo, hi); false: none left (every
+    // further call says so too).  Wave-uniform.
+    __device__ __forceinline__ bool next(uint32_t lane, uint32_t &lo, uint32_t &hi)
+    {
+        uint32_t j = blockIdx.x;
+        if (!first)
+        {
+            uint32_t k = 0;
+            if (waves < chunks && lane == 0) k = atomicAdd(counter, 1u);
+            // wave-uniform (a scalar register), so the loop's exit is
+            // uniform and the compiler keeps no per-lane copies of the
+            // lane state across it
+            j = waves + __builtin_amdgcn_readfirstlane(k);
+        }
+        first = false;
+        const bool some = j < chunks;
+        lo = some ? j * chunk : 0u;
+        hi = some ? min(n, lo + chunk) : 0u;
+        return some;
+    }
+};
+
+// Persistent driver: the launch's waves walk rays [0, n), refilling a wave's
+// idle lanes once `refill` (1..64, wave-uniform) of them wait.  begin(ray, s)
+// starts a ray and returns false if it needs no walk; store(ray, s) writes
+// the result of a completed walk (at the refill that reuses its lane, so the
+// stores of several rays share one pass).  Must be called by every lane of a
 // one-wave block.
 template <bool kCount, bool kTwoLevel, int kShort, uint32_t kChunk, class Begin,
           class Store>
@@ -496,69 +640,75 @@ __device__ __forceinline__ void persistent_walk(SceneView &sv, uint32_t n,
                                                 Store store, Counts &cnt,
                                                 uint32_t &rays)
 {
+    const uint32_t want = walk_waves(n), waves = want < gridDim.x ? want : gridDim.x;
+    if (blockIdx.x >= waves) return;
     __shared__ int lds[kShort * 64];
     const uint32_t lane = threadIdx.x;
     LaneStack<kShort> st{(lint *)lds, (gint *)spill, gridDim.x * 64u,
-                         blockIdx.x * 64u + lane,
-                 lane};
+                         blockIdx.x * 64u + lane, lane};
     const unsigned long long below = (1ull << lane) - 1ull;
+    WorkSource work(counter, n, waves, kChunk);
     uint32_t chunkNext = 0, chunkEnd = 0;
-    bool exhausted = false;
+    bool exhausted = n == 0u;
     uint32_t ray = SPG_MISS;
-    Trav s;
+    // a lane that never gets a ray still runs the steps' straight code: its
+    // state has to be defined (above all the stack pointer, since every lane
+    // writes the slots above its own top)
+    Trav s{};
+    s.cur = kNoStep;
+    s.spBase = -1;
     for (;;)
     {
-        bool need = ray == SPG_MISS;
-        unsigned long long needMask = __ballot(need);
-        const uint32_t idle = (uint32_t)__popcll(needMask);
-        if ((idle >= refill || idle == 64u) && idle != 0u &&
-            !(exhausted && chunkNext >= chunkEnd))
+        const unsigned long long idleMask = __ballot(s.cur == kNoStep);
+        const uint32_t idle = (uint32_t)__popcll(idleMask);
+        const bool more = !(exhausted && chunkNext >= chunkEnd);
+        if (idle == 64u || (idle >= refill && more))
         {
-            if (chunkNext >= chunkEnd)
+            if (s.cur == kNoStep && ray != SPG_MISS)
             {
-                uint32_t base = 0;
-                if (lane == 0) base = atomicAdd(counter, kChunk);
-                // wave-uniform (a scalar register), so the loop's exit is
-                // uniform and the compiler keeps no per-lane copies of the
-                // lane state across it
-                base = __builtin_amdgcn_readfirstlane(base);
-                if (base >= n)
-                {
-                    exhausted = true;
-                    chunkNext = chunkEnd = 0;
-                }
-                else
-                {
-                    chunkNext = base;
-                    chunkEnd = base + kChunk < n ? base + kChunk : n;
-                    if (base + kChunk >= n) exhausted = true;
-                }
+                store(ray, s);
+                ray = SPG_MISS;
+                rays++;
             }
-            uint32_t want = idle;
-            uint32_t avail = chunkEnd - chunkNext;
-            uint32_t rank = (uint32_t)__popcll(needMask & below);
-            if (need && rank < avail)
+            if (!more) break;  // every lane is idle
+            if (chunkNext >= chunkEnd) exhausted = !work.next(lane, chunkNext, chunkEnd);
+            const uint32_t avail = chunkEnd - chunkNext;
+            const uint32_t rank = (uint32_t)__popcll(idleMask & below);
+            if (s.cur == kNoStep && rank < avail)
             {
                 ray = chunkNext + rank;
-                if (!begin(ray, s))
-                {
-                    store(ray, s);
-                    ray = SPG_MISS;
-                    rays++;
-                }
+                if (!begin(ray, s)) s.cur = kNoStep;
             }
-            chunkNext += want < avail ? want : avail;
+            chunkNext += idle < avail ? idle : avail;
         }
-        // one path round the loop: with no active lane the step's branches
-        // are all skipped, and the lane state needs no copies for a second
-        // path back to the loop head
-        if (__ballot(ray != SPG_MISS) == 0ull && exhausted && chunkNext >= chunkEnd)
-            break;
-        if (trav_step<kCount, kTwoLevel, kShort>(sv, s, st, cnt, ray != SPG_MISS))
+        // The kind of step this iteration runs: the lanes of each kind are
+        // counted and the largest weighted count wins; the other lanes wait.
+        const bool isNode = (uint32_t)s.cur < kFirstStepCode;
+        const unsigned long long mNode = __ballot(isNode);
+        const unsigned long long mLeaf = __ballot(s.cur < 0);
+        if (kTwoLevel)
         {
-            store(ray, s);
-            ray = SPG_MISS;
-            rays++;
+            const unsigned long long mIn = __ballot(s.spBase >= 0);
+            const unsigned long long mFin = __ballot(s.cur == kFinishStep);
+            const int wNode = __popcll(mNode) * kNodeWeight,
+                      wTri = __popcll(mLeaf & mIn) * kTriangleWeight,
+                      wEnter = __popcll(mLeaf & ~mIn) * kEnterWeight,
+                      wFin = __popcll(mFin) * kFinishWeight;
+            if (wNode >= wTri && wNode >= wEnter && wNode >= wFin)
+                step_node<kCount, true>(sv, s, st, cnt, isNode);
+            else if (wTri >= wEnter && wTri >= wFin)
+                step_triangle<kCount, true>(sv, s, st, cnt, s.cur < 0 && s.spBase >= 0);
+            else if (wEnter >= wFin)
+                step_enter<kCount>(sv, s, cnt, s.cur < 0 && s.spBase < 0);
+            else
+                step_finish(sv, s, st, s.cur == kFinishStep);
+        }
+        else
+        {
+            if (__popcll(mNode) * kNodeWeight >= __popcll(mLeaf) * kTriangleWeight)
+                step_node<kCount, false>(sv, s, st, cnt, isNode);
+            else
+                step_triangle<kCount, false>(sv, s, st, cnt, s.cur < 0);
         }
     }
 }
