@@ -331,7 +331,9 @@ int spg_time_intersect_closest(spg_Scene *scene, uint32_t meshId,
                                double *meanKernelMs);
 /* Kernel timings of the last trace call on this device, in ms, summed over
  * its launches: [0] raygen [1] extend [2] shade [3] finalize [4] guide
- * [5] total wall; launches[i] counts launches. */
+ * [5] total wall; launches[i] counts launches.  A launch's time runs to the
+ * start of the next one; of calls of more than 512 launches the first 511
+ * are timed (the total and the counts cover all). */
 int spg_last_trace_timings(spg_Device *dev, double *ms6, uint32_t *launches6);
 /* Raw counters of the last trace call on this device: [0] rays [1] hits
  * [2] misses [3] mesh-hierarchy slab tests [4] mesh (instance) entries

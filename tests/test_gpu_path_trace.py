@@ -332,3 +332,26 @@ def test_slot_list_cache_invalidation(device):
         assert np.array_equal(r.view(np.uint32), fresh[key].view(np.uint32))
     s_big.close()
     s_small.close()
+
+
+@pytest.mark.parametrize("spp", [1, 2, 60])
+def test_passes_and_launch_times(device, spp):
+    """One sample per pass: the first pass starts the sums, the last writes
+    the pixels (1: both at once), and 60 passes of 12 launches are more than
+    the launch times kept per call.  Image bit-exact against the oracle;
+    class times add up to at most the total.
+    An empty tile list after it reports no rays."""
+    desc = scenes.config1(16, 8, env="cube", env_size=16)
+    img, m = gpu_render(device, desc, spp, 5, V.EST_PARITY, V.RNG_XORSHIFT_PIXEL)
+    want, met = oracle_render(desc, spp, 5, V.EST_PARITY, SPO_RNG_XORSHIFT_PIXEL)
+    assert np.array_equal(img.view(np.uint32), want.view(np.uint32))
+    assert [m.values[k] for k in (1, 2, 3, 4)] == [int(met[k]) for k in (1, 2, 3, 4)]
+    t = device.last_timings()
+    classes = sum(t[k][0] for k in t if k != "total")
+    # (sums of the same 10 ns ticks: equal up to the rounding of doubles)
+    assert 0.0 < classes <= t["total"][0] * (1 + 1e-9)
+    assert t["raygen"][1] == t["finalize"][1] == spp and t["extend"][1] == 5 * spp
+    s, cam = scenes.load_gpu(device, desc)
+    ctx = V.make_context(cam, s, spp=spp, bounces=5, estimator=V.EST_PARITY, collect=True)
+    m2 = V.path_trace_tiles(ctx, [], np.zeros(16 * 8 * 4, np.float32))
+    assert m2.values[V.METRIC_RAYS] == 0

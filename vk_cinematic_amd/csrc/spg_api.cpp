@@ -172,6 +172,23 @@ int spg_device_create(int ordinal, spg_Device **out)
         delete d;
         return hip_check(e, "hipMalloc(traversal spill)");
     }
+    int khz = 0;
+    e = hipHostMalloc((void **)&d->report, sizeof(TraceReport), hipHostMallocDefault);
+    if (e == hipSuccess)
+        e = hipMalloc((void **)&d->stamps, kStamps * sizeof(unsigned long long));
+    if (e == hipSuccess)
+        e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ordinal);
+    if (e != hipSuccess)
+    {
+        for (int i = 0; i < kEvents; ++i) hipEventDestroy(d->ev[i]);
+        hipStreamDestroy(d->stream);
+        hipFree(d->persistBlock);
+        if (d->report) hipHostFree(d->report);
+        if (d->stamps) hipFree(d->stamps);
+        delete d;
+        return hip_check(e, "trace report buffers");
+    }
+    if (khz > 0) d->clockKHz = khz;
     d->persist.counter = (uint32_t *)d->persistBlock;
     d->persist.spill = (int *)((char *)d->persistBlock + 256);
     // the allocation-free entry point's scratch: this device's copy of the
@@ -182,6 +199,8 @@ int spg_device_create(int ordinal, spg_Device **out)
         for (int i = 0; i < kEvents; ++i) hipEventDestroy(d->ev[i]);
         hipStreamDestroy(d->stream);
         hipFree(d->persistBlock);
+        hipHostFree(d->report);
+        hipFree(d->stamps);
         delete d;
         return hip_check(e, "hipGetSymbolAddress(scratch)");
     }
@@ -201,8 +220,9 @@ static void delete_device(spg_Device *d)
     hipSetDevice(d->ordinal);
     hipStreamSynchronize(d->stream);
     free_paths(d);
-    free_ptr(d->image);
     if (d->hostStage) hipHostFree(d->hostStage);
+    if (d->report) hipHostFree(d->report);
+    if (d->stamps) hipFree(d->stamps);
     free_ptr(d->slotPixel);
     free_ptr(d->accum);
     free_ptr(d->persistBlock);
@@ -1100,28 +1120,8 @@ static int ensure_buffer(void *&ptr, size_t &have, size_t count)
     return SPG_OK;
 }
 
-struct LaunchTimer
-{
-    spg_Device *d;
-    int next = 0;
-    int cls[(kEvents - 4) / 2];
-    bool on = true;
-    void begin(int c)
-    {
-        if (!on || next >= kEvents - 4) return;
-        cls[next / 2] = c;
-        hipEventRecord(d->ev[next], d->stream);
-    }
-    void end()
-    {
-        if (!on || next >= kEvents - 4) return;
-        hipEventRecord(d->ev[next + 1], d->stream);
-        next += 2;
-    }
-};
-
-// devImage == nullptr: render into the device's staging image (sized here,
-// under the device lock) and copy the tiles out to hostImage.
+// devImage == nullptr: the pixels go to the device's pinned staging buffer
+// (sized here, under the device lock), then tile by tile to hostImage.
 static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
                  spg_Metrics *metrics, float *devImage, float *hostImage)
 {
@@ -1181,13 +1181,11 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
     const std::vector<uint32_t> &slots = d->slots;
     if (!devImage)
     {
-        // host pixels: the tiles' pixels gathered in slot order on the
-        // device, then one copy into pinned host memory and a scatter of
-        // the tile rows into the caller's image (a strided copy per tile
-        // into pageable memory costs a runtime round trip per row)
+        // host pixels: the last launch of a slot chunk writes its pixels in
+        // slot order straight into pinned host memory, and the tile rows are
+        // scattered from there into the caller's image (a strided copy per
+        // tile into pageable memory costs a runtime round trip per row)
         const size_t bytes = std::max<size_t>(slots.size(), 1) * 16;
-        CHK(ensure_buffer<float>(d->image, d->imageCount, bytes / 4));
-        devImage = (float *)d->image;
         if (d->hostStageBytes < bytes)
         {
             if (d->hostStage) hipHostFree(d->hostStage);
@@ -1208,7 +1206,6 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
     CHK(ensure_buffer<uint32_t>(d->slotPixel, d->slotPixelCount, cap));
     if (d->slotPixelCount != slotHave) d->slotsOnDevice = false;  // reallocated
     CHK(ensure_buffer<float>(d->accum, d->accumCount, 3 * (size_t)cap));
-    HIPCHK(launch_clear_counters(d->stream, (uint32_t *)d->paths.metrics, 32));
 
     TraceParams p{};
     p.scene = s->dev_scene;
@@ -1225,6 +1222,8 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
     p.tx = cfg.transcendentals;
     p.collect = cfg.collectMetrics;
     p.work = d->persist.counter;
+    p.stamps = d->stamps;
+    p.firstLaunch = 1u;
     const bool train = guided && cfg.guideTrain;
     if (guided)
         CHK(guide_prepare_trace(cfg.guide, s, cap, cfg.bounces, train, p.guide));
@@ -1245,9 +1244,17 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
             p.scene.envSelect = light_split(s->lightStat, p.scene.envSelect);
     }
 
-    LaunchTimer tm{d};
     uint32_t launches[6] = {0};
-    hipEventRecord(d->ev[kEvents - 2], d->stream);
+    // the kernel class of each stamped launch, in order; training kernels
+    // run between the sample collection's stamp and the next launch's
+    uint8_t cls[kStamps];
+    uint32_t begun = 0;
+    auto begin = [&](int c) {
+        p.stamp = std::min(begun, kStamps);
+        if (begun < kStamps) cls[begun] = (uint8_t)c;
+        ++begun;
+        launches[c]++;
+    };
     for (size_t s0 = 0; s0 < slots.size(); s0 += cap)
     {
         uint32_t nslots = (uint32_t)std::min<size_t>(cap, slots.size() - s0);
@@ -1256,14 +1263,17 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
             HIPCHK(hipMemcpyAsync(d->slotPixel, slots.data() + s0, 4 * (size_t)nslots,
                                   hipMemcpyHostToDevice, d->stream));
         d->slotsOnDevice = whole;
-        HIPCHK(launch_clear_floats(d->stream, p.accum, 3 * (size_t)nslots));
         p.slots = nslots;
+        p.image = hostImage ? nullptr : devImage;
+        p.slotOut = hostImage ? (float *)d->hostStage + 4 * s0 : nullptr;
         uint32_t sppPass = pcg ? std::max(1u, std::min(spp, cap / nslots)) : 1u;
         for (uint32_t done = 0; done < spp;)
         {
             uint32_t sp = std::min(sppPass, spp - done);
             p.sppPass = sp;
             p.sampleBase = cfg.sampleOffset + done;
+            p.firstPass = done == 0 ? 1u : 0u;
+            p.lastPass = done + sp >= spp ? 1u : 0u;
             // accum and the paths are laid out with the slot count of this
             // chunk; accum rows are 3 x nslots
             if (guided)
@@ -1271,69 +1281,50 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
                                      (p.sampleBase + 1u) * 0x9E3779B9u ^ cfg.seed ^
                                          (uint32_t)s0,
                                      nslots * sp));
-            tm.begin(kRaygen);
+            begin(kRaygen);
             HIPCHK(launch_raygen(d->stream, p));
-            tm.end();
-            launches[kRaygen]++;
+            p.firstLaunch = 0u;
             int q = 0;
             for (uint32_t b = 0; b < cfg.bounces; ++b)
             {
-                tm.begin(kExtend);
+                begin(kExtend);
                 HIPCHK(launch_extend(d->stream, p, q, d->persist));
-                tm.end();
                 // at the last bounce no hit scatters (a path at bounce b
                 // holds b vertices), so there is nothing to infer
                 if (guided && b + 1 < cfg.bounces)
                 {
-                    tm.begin(kGuide);
+                    begin(kGuide);
                     HIPCHK(launch_guide_infer(d->stream, p, q));
-                    tm.end();
-                    launches[kGuide]++;
                 }
-                tm.begin(kShade);
+                begin(kShade);
                 HIPCHK(launch_shade(d->stream, p, q));
-                tm.end();
-                launches[kExtend]++;
-                launches[kShade]++;
                 if (nee && b + 1 < cfg.bounces)
                 {
                     // shadow rays of this bounce, then their contributions
-                    tm.begin(kExtend);
+                    begin(kExtend);
                     HIPCHK(launch_extend(d->stream, p, 2, d->persist));
-                    tm.end();
-                    tm.begin(kShade);
+                    begin(kShade);
                     HIPCHK(launch_resolve_shadow(d->stream, p));
-                    tm.end();
-                    launches[kExtend]++;
-                    launches[kShade]++;
                 }
                 q ^= 1;
             }
-            tm.begin(kFinal);
+            begin(kFinal);
             HIPCHK(launch_finalize(d->stream, p));
-            tm.end();
-            launches[kFinal]++;
             if (train)
             {
-                tm.begin(kGuide);
+                begin(kGuide);
                 HIPCHK(launch_guide_collect(d->stream, p));
                 CHK(guide_train_pass(cfg.guide, d->stream));
-                tm.end();
-                launches[kGuide]++;
             }
             done += sp;
         }
-        if (hostImage) HIPCHK(launch_write_slots(d->stream, p, devImage + 4 * s0));
-        else HIPCHK(launch_write_pixels(d->stream, p, devImage));
     }
-    hipEventRecord(d->ev[kEvents - 1], d->stream);
     unsigned long long m[16] = {0};
-    HIPCHK(hipMemcpyAsync(m, d->paths.metrics, 128, hipMemcpyDeviceToHost,
-                          d->stream));
-    if (hostImage && !slots.empty())
-        HIPCHK(hipMemcpyAsync(d->hostStage, devImage, slots.size() * 16,
-                              hipMemcpyDeviceToHost, d->stream));
+    const uint32_t stamped = std::min(begun, kStamps);
+    if (begun)
+        HIPCHK(launch_report(d->stream, d->paths, d->stamps, stamped, d->report));
     HIPCHK(hipStreamSynchronize(d->stream));
+    if (begun) memcpy(m, d->report->metrics, sizeof m);
     if (p.learnLight)
     {
         uint64_t *stat = cfg.estimator == SPG_EST_GUIDED_NEE ? cfg.guide->lightStat
@@ -1359,15 +1350,16 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
     }
     auto t1 = std::chrono::steady_clock::now();
     for (int k = 0; k < 6; ++k) d->lastMs[k] = 0.0;
-    for (int k = 0; k < tm.next; k += 2)
+    const TraceReport &rep = *d->report;
+    for (uint32_t k = 0; k < stamped; ++k)
     {
-        float ms = 0.0f;
-        hipEventElapsedTime(&ms, d->ev[k], d->ev[k + 1]);
-        d->lastMs[tm.cls[k / 2]] += ms;
+        // a stamp's interval ends at the next one, the last launch's at the
+        // report (beyond kStamps launches the rest is not timed by class)
+        if (k + 1 == stamped && begun > stamped) break;
+        const unsigned long long end = k + 1 < stamped ? rep.stamps[k + 1] : rep.end;
+        d->lastMs[cls[k]] += (double)(end - rep.stamps[k]) / d->clockKHz;
     }
-    float total = 0.0f;
-    hipEventElapsedTime(&total, d->ev[kEvents - 2], d->ev[kEvents - 1]);
-    d->lastMs[5] = total;
+    if (stamped) d->lastMs[5] = (double)(rep.end - rep.stamps[0]) / d->clockKHz;
     for (int k = 0; k < 6; ++k) d->lastLaunches[k] = launches[k];
     for (int k = 0; k < 8; ++k) d->lastCounters[k] = m[k];
     if (metrics)

@@ -152,8 +152,9 @@ int record(spg_Batch *b, hipStream_t st, const spg_TraceConfig &cfg,
     p.learnLight = cfg.estimator == SPG_EST_GUIDED_NEE && train ? 1u : 0u;
     b->learnLight = p.learnLight != 0;
     uint32_t k = 0;
-    HIPCHK(launch_clear_counters(st, (uint32_t *)b->paths.metrics, 32));
-    ++k;
+    if (b->slots == 0) HIPCHK(launch_clear_counters(st, (uint32_t *)b->paths.metrics, 32));
+    p.firstLaunch = 1u;
+    p.stamp = kStamps;  // launches carry no stamps (profiles time them with events)
     const bool pcg = cfg.rngMode == SPG_RNG_PCG;
     const uint32_t spp = cfg.samplesPerPixel;
     for (uint64_t s0 = 0; s0 < b->slots; s0 += cap)
@@ -162,14 +163,14 @@ int record(spg_Batch *b, hipStream_t st, const spg_TraceConfig &cfg,
         p.slotPixel = b->dSlotPixel + s0;
         p.slotItem = b->dSlotItem + s0;
         p.slots = nslots;
-        HIPCHK(launch_clear_floats(st, p.accum, 3 * (size_t)nslots));
-        ++k;
         uint32_t sppPass = pcg ? std::max(1u, std::min(spp, cap / nslots)) : 1u;
         for (uint32_t done = 0; done < spp;)
         {
             uint32_t sp = std::min(sppPass, spp - done);
             p.sppPass = sp;
             p.sampleBase = cfg.sampleOffset + done;
+            p.firstPass = done == 0 ? 1u : 0u;
+            p.lastPass = done + sp >= spp ? 1u : 0u;
             if (guided)
             {
                 // the same pass salt as an eager trace of these slots
@@ -182,6 +183,7 @@ int record(spg_Batch *b, hipStream_t st, const spg_TraceConfig &cfg,
             CHK(T0(kRaygen));
             HIPCHK(launch_raygen(st, p));
             CHK(T1());
+            p.firstLaunch = 0u;
             ++k;
             int q = 0;
             for (uint32_t bb = 0; bb < cfg.bounces; ++bb)
@@ -228,8 +230,6 @@ int record(spg_Batch *b, hipStream_t st, const spg_TraceConfig &cfg,
             }
             done += sp;
         }
-        HIPCHK(launch_write_pixels(st, p, nullptr));
-        ++k;
     }
     if (kernels) *kernels = k;
     return SPG_OK;

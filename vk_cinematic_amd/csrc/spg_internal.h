@@ -211,6 +211,16 @@ struct TraceParams
     DevPaths paths;
     const uint32_t *slotPixel;   // pixel index of each slot
     float *accum;                // [3][slots] running sums (sample order)
+    // the slot chunk's first / last pass: the sums start at zero / the pixels
+    // are written (the caller's image by pixel, `slotOut` by slot; a batch
+    // writes its items' images)
+    uint32_t firstPass, lastPass;
+    float *image, *slotOut;
+    uint32_t firstLaunch;        // the call's first pass: zero the metrics
+    // launch start times (device clock), written at stamps[stamp] by the
+    // launch's first block; stamp >= kStamps: not recorded
+    unsigned long long *stamps;
+    uint32_t stamp;
     uint32_t slots;
     uint32_t sppPass;            // samples of each slot in this pass
     uint32_t sampleBase;         // first sample index of this pass
@@ -234,6 +244,16 @@ struct TraceParams
     const DevScene *scenes;
     const DevCamera *cams;
     float *const *images;
+};
+
+constexpr uint32_t kStamps = 512;
+// What a trace call reports to the host (pinned memory, written by its last
+// launch): the metrics, the device time of that launch, the launch stamps.
+struct TraceReport
+{
+    unsigned long long metrics[16];
+    unsigned long long end;
+    unsigned long long stamps[kStamps];
 };
 
 // Loss scale of the FP16 gradients in guide training.
@@ -268,10 +288,9 @@ struct GuideAdam
 
 }  // namespace spg
 
-// HIP events per device: timed intervals of a trace use [0, kEvents - 4),
-// the trace total the last two, a closest-hit timing the two before; the
-// post-step timing uses kEvents - 4 .. kEvents - 2 (each call reads its
-// events before returning, under the device lock).
+// HIP events per device: a batch profile's timed intervals use
+// [0, kEvents - 4), a closest-hit timing and the post-step timing the last
+// four (each call reads its events before returning, under the device lock).
 constexpr int kEvents = 256;
 
 // One caller's host-pixel trace waiting to be combined with other callers'
@@ -308,10 +327,11 @@ struct spg_Device
     spg::DevPaths paths{};
     size_t pathsBytes = 0;
     void *pathsBlock = nullptr;
-    void *image = nullptr;       // host-pixel calls: the tiles' pixels in
-    size_t imageCount = 0;       // slot order (RGBA32F per slot)
-    void *hostStage = nullptr;   // pinned host copy of `image`
-    size_t hostStageBytes = 0;
+    void *hostStage = nullptr;   // host-pixel calls: the tiles' pixels in slot
+    size_t hostStageBytes = 0;   // order (RGBA32F), pinned, written by the device
+    spg::TraceReport *report = nullptr; // pinned, written by the device
+    unsigned long long *stamps = nullptr; // device, [kStamps]
+    double clockKHz = 1e5;       // the device clock's rate
     void *slotPixel = nullptr;   // pixel index per slot
     size_t slotPixelCount = 0;
     // the slot list of the last trace call (pixels of its tiles in tile
@@ -485,10 +505,9 @@ hipError_t launch_resolve_shadow(hipStream_t s, const TraceParams &p);
 hipError_t launch_finalize(hipStream_t s, const TraceParams &p);
 // guided training: the pass's samples in a fixed order (after finalize)
 hipError_t launch_guide_collect(hipStream_t s, const TraceParams &p);
-hipError_t launch_write_pixels(hipStream_t s, const TraceParams &p,
-                               float *image);
-// the pass's pixels in slot order: out[slot] (single-scene launches)
-hipError_t launch_write_slots(hipStream_t s, const TraceParams &p, float *out);
+// the call's metrics and its first `stamps` launch stamps to the host
+hipError_t launch_report(hipStream_t s, const DevPaths &paths,
+                         const unsigned long long *stamps, uint32_t n, TraceReport *out);
 hipError_t launch_clear_counters(hipStream_t s, uint32_t *counters, int n);
 hipError_t launch_set_counter(hipStream_t s, uint32_t *counter, uint32_t v);
 hipError_t launch_clear_floats(hipStream_t s, float *p, size_t n);

@@ -26,6 +26,16 @@ __device__ __forceinline__ uint32_t lane_id()
     return __lane_id();
 }
 
+// The launch's start time, for the call's timings: kernels of a stream run
+// back to back, so the difference of two launches' stamps is the first one's
+// time.  (Event records between the launches would each stop the stream for
+// about 5 us.)
+__device__ __forceinline__ void stamp_launch(const TraceParams &p)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.stamp < kStamps)
+        p.stamps[p.stamp] = wall_clock64();
+}
+
 // Sum over the active lanes of the wave, result valid in every lane.
 __device__ __forceinline__ unsigned long long wave_sum(unsigned long long x)
 {
@@ -673,6 +683,8 @@ template <bool kBatch>
 __global__ __launch_bounds__(256) void k_raygen(TraceParams p)
 {
     const uint32_t nPaths = p.slots * p.sppPass;
+    stamp_launch(p);
+    if (p.firstLaunch && blockIdx.x == 0 && threadIdx.x < 16) p.paths.metrics[threadIdx.x] = 0ull;
     if (blockIdx.x == 0 && threadIdx.x == 0)
     {
         // this pass's camera rays fill queue 0; the first k_extend starts
@@ -757,6 +769,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_extend(TraceParams p, int q,
                                                         int *spill)
 {
     const uint32_t n = p.paths.counters[q];
+    stamp_launch(p);
     const uint32_t cap = p.paths.capacity;
     const float *qo = p.paths.qo[q], *qd = p.paths.qd[q];
     if (!kShadow && blockIdx.x == 0 && threadIdx.x == 0)
@@ -1009,6 +1022,7 @@ template <bool kDouble, int kEst, bool kBatch>
 __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
 {
     const uint32_t n = p.paths.counters[q];
+    stamp_launch(p);
     // k_extend has finished with the work counter: zero it for the next one
     if (blockIdx.x == 0 && threadIdx.x == 0) *p.work = 0u;
     const uint32_t cap = p.paths.capacity;
@@ -1345,6 +1359,7 @@ __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
 __global__ __launch_bounds__(256) void k_resolve_shadow(TraceParams p)
 {
     const uint32_t n = p.paths.counters[2];
+    stamp_launch(p);
     if (blockIdx.x == 0 && threadIdx.x == 0) *p.work = 0u;  // for the next k_extend
     const uint32_t cap = p.paths.capacity;
     unsigned long long lum[2] = {0ull, 0ull};  // learned light split: sky, emitters
@@ -1433,11 +1448,13 @@ __global__ __launch_bounds__(256) void k_finalize(TraceParams p)
 {
     const uint32_t cap = p.paths.capacity;
     const float invSpp = 1.0f / (float)p.spp;
+    stamp_launch(p);
     for (uint32_t slot = xcd_block() * 256 + threadIdx.x; slot < p.slots;
          slot += gridDim.x * 256)
     {
-        v3 total{p.accum[slot], p.accum[p.slots + slot],
-                 p.accum[2 * p.slots + slot]};
+        v3 total{0.0f, 0.0f, 0.0f};
+        if (!p.firstPass)
+            total = v3{p.accum[slot], p.accum[p.slots + slot], p.accum[2 * p.slots + slot]};
         uint32_t lastXs = 0;
         for (uint32_t k = 0; k < p.sppPass; ++k)
         {
@@ -1475,9 +1492,22 @@ __global__ __launch_bounds__(256) void k_finalize(TraceParams p)
             total = total + radiance * invSpp;
             lastXs = p.paths.rngXs[path];
         }
-        p.accum[slot] = total.x;
-        p.accum[p.slots + slot] = total.y;
-        p.accum[2 * p.slots + slot] = total.z;
+        if (p.lastPass)
+        {
+            // the chunk's pixels, alpha 1: by slot (tile order) for the
+            // host-pixel calls, whose tile rows are runs of slots, else by
+            // pixel
+            float4 *dst = reinterpret_cast<float4 *>(
+                p.slotOut ? p.slotOut : p.slotItem ? p.images[p.slotItem[slot]] : p.image);
+            dst[p.slotOut ? slot : p.slotPixel[slot]] =
+                make_float4(total.x, total.y, total.z, 1.0f);
+        }
+        else
+        {
+            p.accum[slot] = total.x;
+            p.accum[p.slots + slot] = total.y;
+            p.accum[2 * p.slots + slot] = total.z;
+        }
         if (p.rngMode != SPG_RNG_PCG) p.paths.slotRng[slot] = lastXs;
     }
 }
@@ -1521,6 +1551,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan_1024(uint32_t x, uint32
 __global__ __launch_bounds__(1024) void k_gscan_sums(TraceParams p)
 {
     __shared__ uint32_t sh[40];
+    stamp_launch(p);
     const uint32_t N = p.slots * p.sppPass;
     const uint32_t v0 = blockIdx.x * kGScanSeg + threadIdx.x * 4;
     uint32_t c = 0;
@@ -1588,6 +1619,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_guide_infer(TraceParams p,
     __shared__ _Float16 sW[kWLdsHalves];
     __shared__ float sBias[kGRows];
     __shared__ float waveOut[kInferWaves][kTileScratchFloats];
+    stamp_launch(p);
     stage_rows(sW, p.guide.w16, kGRows);
     for (int k = threadIdx.x; k < kGRows; k += blockDim.x) sBias[k] = p.guide.bias[k];
     __syncthreads();
@@ -1639,29 +1671,15 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_guide_infer(TraceParams p,
     if (lane == 0 && evals) atomicAdd(&p.paths.metrics[7], evals);
 }
 
-template <bool kBatch>
-__global__ void k_write_pixels(TraceParams p, float *image)
+// The call's last launch: counters and launch stamps into pinned host memory
+// (no separate copies), with its own time as the end of the call.
+__global__ __launch_bounds__(64) void k_report(const unsigned long long *metrics,
+                                               const unsigned long long *stamps, uint32_t n,
+                                               TraceReport *out)
 {
-    for (uint32_t slot = blockIdx.x * 256 + threadIdx.x; slot < p.slots;
-         slot += gridDim.x * 256)
-    {
-        uint32_t pixel = p.slotPixel[slot];
-        float4 c = make_float4(p.accum[slot], p.accum[p.slots + slot],
-                               p.accum[2 * p.slots + slot], 1.0f);
-        float *dst = kBatch ? p.images[p.slotItem[slot]] : image;
-        reinterpret_cast<float4 *>(dst)[pixel] = c;
-    }
-}
-
-// Host-pixel calls: the chunk's pixels in slot order (tile order), so one
-// contiguous copy brings every tile to the host.
-__global__ void k_write_slots(TraceParams p, float *out)
-{
-    for (uint32_t slot = blockIdx.x * 256 + threadIdx.x; slot < p.slots;
-         slot += gridDim.x * 256)
-        reinterpret_cast<float4 *>(out)[slot] =
-            make_float4(p.accum[slot], p.accum[p.slots + slot],
-                        p.accum[2 * p.slots + slot], 1.0f);
+    if (threadIdx.x == 0) out->end = wall_clock64();
+    if (threadIdx.x < 16) out->metrics[threadIdx.x] = metrics[threadIdx.x];
+    for (uint32_t i = threadIdx.x; i < n; i += 64) out->stamps[i] = stamps[i];
 }
 
 __global__ void k_clear_u32(uint32_t *p, int n)
@@ -1975,22 +1993,10 @@ hipError_t launch_guide_collect(hipStream_t s, const TraceParams &p)
     return hipGetLastError();
 }
 
-hipError_t launch_write_pixels(hipStream_t s, const TraceParams &p,
-                               float *image)
+hipError_t launch_report(hipStream_t s, const DevPaths &paths,
+                         const unsigned long long *stamps, uint32_t n, TraceReport *out)
 {
-    if (p.slotItem)
-        hipLaunchKernelGGL(k_write_pixels<true>, dim3(grid_for(p.slots, 256, 4096)),
-                           dim3(256), 0, s, p, image);
-    else
-        hipLaunchKernelGGL(k_write_pixels<false>, dim3(grid_for(p.slots, 256, 4096)),
-                           dim3(256), 0, s, p, image);
-    return hipGetLastError();
-}
-
-hipError_t launch_write_slots(hipStream_t s, const TraceParams &p, float *out)
-{
-    hipLaunchKernelGGL(k_write_slots, dim3(grid_for(p.slots, 256, 4096)), dim3(256), 0, s,
-                       p, out);
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s, paths.metrics, stamps, n, out);
     return hipGetLastError();
 }
 
