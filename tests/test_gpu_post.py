@@ -52,3 +52,22 @@ def test_progressive_accumulation(device):
     for buf in (acc, part, full):
         buf.free()
     s.close()
+
+
+@pytest.mark.parametrize("pixels", [1, 255, 257, 2048 * 256 + 3])
+def test_tonemap_bytes_at_every_step(device, pixels):
+    """Radiances around each of the 255 steps of the byte (the floats within
+    40 of the step's preimage c = x / (1 - x), x = ((k - 1/2) / 255)^2.2), and
+    the values outside [0, 1): the oracle's bytes exactly."""
+    x = ((np.arange(1, 256) - 0.5) / 255.0) ** 2.2
+    c = (x / (1.0 - x)).astype(np.float32).view(np.int32)
+    near = (c[:, None] + np.arange(-40, 41)).astype(np.int32).ravel().view(np.float32)
+    odd = np.array([0.0, -0.0, 1e-45, 1e-38, 3e38, np.inf, -np.inf, np.nan, -0.5, -1.0,
+                    -2.0, -1e-45, -3e38, 2.0 ** 24, 2.0 ** 25, 1.0], np.float32)
+    px = np.resize(np.concatenate([odd, near]), pixels * 4).astype(np.float32)
+    img = device.alloc(pixels * 16)
+    img.upload(px)
+    for exposure in (1.0, 2.0, -1.0):
+        got = device.tonemap(img, pixels, exposure, V.TX_DOUBLE)
+        assert np.array_equal(got, _tonemap(px, exposure, SPO_TX_CR))
+    img.free()
