@@ -60,7 +60,22 @@ __device__ __forceinline__ void cube_basis(uint32_t face, v3 &fwd, v3 &up, v3 &r
 
 // One wave per texel of 6 faces of w x h.  phis / thetas hold the values
 // the reference's float loop counters take (phi += 0.1f below 2 pi, theta
-// += 0.1f below pi/2); sample k is (phis[k / nTheta], thetas[k % nTheta]).
+// += 0.1f below pi/2: 63 and 16, at most kIrrGrid together); sample k is
+// (phis[k / nTheta], thetas[k % nTheta]).
+//
+// Bound by the gathers (four texels per sample, nearly every sample in lines
+// of its own; the source exceeds an XCD's L2), then by the double-precision
+// transcendentals and the chain of additions.  Of the seven transcendentals
+// per sample (sine and cosine of both angles, two arc tangents, a cosine) the
+// four of the grid's angles are evaluated once per block into LDS, the same
+// functions of the same floats.  The chain adds a batch's 64 values from
+// registers (with one LDS read per addition each waited for its read).  An
+// XCD's texels are neighbours, so its L2 holds the hemisphere they share.
+// 6 x 32 x 32 texels of a 1024 x 512 source: 126 -> 89 us (107 with the
+// table, 91 with the register chain); 6 x 8 x 8: 39 -> 29; 6 x 64 x 64 of
+// 2048 x 1024: 578 -> 573.  A budget of 6 waves per SIMD spills (144 us).
+constexpr uint32_t kIrrGrid = 128;
+constexpr int kIrrRow = 68;  // the three rows start in different LDS banks
 template <bool kDouble>
 __global__ __launch_bounds__(64 * kIrrWaves) void k_irradiance(
     const float4 *__restrict__ src, uint32_t ew, uint32_t eh, uint32_t w,
@@ -68,9 +83,20 @@ __global__ __launch_bounds__(64 * kIrrWaves) void k_irradiance(
     const float *__restrict__ thetas, uint32_t nTheta, float clampValue,
     float4 *__restrict__ out)
 {
-    __shared__ float part[kIrrWaves][3][64];
+    __shared__ __align__(16) float part[kIrrWaves][3][kIrrRow];
+    __shared__ float sine[kIrrGrid], cosine[kIrrGrid];
+    for (uint32_t k = threadIdx.x; k < nPhi + nTheta; k += 64 * kIrrWaves)
+    {
+        const float a = k < nPhi ? phis[k] : thetas[k - nPhi];
+        sine[k] = Tx<kDouble>::sin_(a);
+        cosine[k] = Tx<kDouble>::cos_(a);
+    }
+    __syncthreads();
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t texel = blockIdx.x * kIrrWaves + wave;
+    // consecutive texels on one XCD (blocks go to the 8 XCDs in turn; the
+    // grid is a multiple of 8)
+    const uint32_t texel =
+        ((blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u) * kIrrWaves + wave;
     if (texel >= 6u * w * h) return;  // whole waves; no block barrier below
     const uint32_t face = texel / (w * h), rem = texel % (w * h);
     const uint32_t y = rem / w, x = rem % w;
@@ -90,13 +116,13 @@ __global__ __launch_bounds__(64 * kIrrWaves) void k_irradiance(
     for (uint32_t base = 0; base < count; base += 64)
     {
         const uint32_t k = base + lane;
-        v3 c{0.0f, 0.0f, 0.0f};
+        v3 c{-0.0f, -0.0f, -0.0f};  // past the end: adding it changes nothing
         if (k < count)
         {
-            const float phi = phis[k / nTheta], theta = thetas[k % nTheta];
+            const uint32_t phi = k / nTheta, theta = nPhi + k % nTheta;
             // MapSphericalToCartesianCoordinates, src/math_lib.h:864-871
-            const float st = Tx<kDouble>::sin_(theta), ct = Tx<kDouble>::cos_(theta);
-            const v3 td{st * Tx<kDouble>::cos_(phi), ct, st * Tx<kDouble>::sin_(phi)};
+            const float st = sine[theta], ct = cosine[theta];
+            const v3 td{st * cosine[phi], ct, st * sine[phi]};
             const v3 wd = (n * td.y + t * td.x) + b * td.z;
             // ToSphericalCoordinates + MapToEquirectangular,
             // src/math_lib.h:849-884, v flipped
@@ -117,9 +143,13 @@ __global__ __launch_bounds__(64 * kIrrWaves) void k_irradiance(
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (lane < 3)
         {
-            const uint32_t m = count - base < 64u ? count - base : 64u;
-            const float *row = mine + lane * 64;
-            for (uint32_t j = 0; j < m; ++j) acc += row[j];
+            const float4 *row = reinterpret_cast<const float4 *>(mine + lane * kIrrRow);
+            float4 v[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) v[j] = row[j];
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                acc = (((acc + v[j].x) + v[j].y) + v[j].z) + v[j].w;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -137,8 +167,9 @@ hipError_t launch_irradiance(hipStream_t s, const float4 *src, uint32_t ew,
                              uint32_t nPhi, const float *thetas, uint32_t nTheta,
                              float clampValue, bool dbl, float4 *out)
 {
+    if (nPhi + nTheta > kIrrGrid) return hipErrorInvalidValue;
     const uint32_t texels = 6u * w * h;
-    const uint32_t blocks = (texels + kIrrWaves - 1) / kIrrWaves;
+    const uint32_t blocks = (texels + 8 * kIrrWaves - 1) / (8 * kIrrWaves) * 8;
     if (dbl)
         k_irradiance<true><<<blocks, 64 * kIrrWaves, 0, s>>>(
             src, ew, eh, w, h, phis, nPhi, thetas, nTheta, clampValue, out);
