@@ -233,3 +233,25 @@ def test_full_size_guided_workload_properties(device, name):
     g.close()
     dimg.free()
     s.close()
+
+
+@pytest.mark.parametrize("W,H", [(1, 1), (33, 31), (41, 25), (65, 63), (241, 17)])
+def test_training_samples_at_segment_edges(device, W, H):
+    """Path counts of one, one less and one more than a block of the sample
+    export (1024 paths) and than a segment of its scan (4096): every
+    candidate sample of the oracle once, bit for bit."""
+    desc = scenes.config1(W, H, env="cube", env_size=32)
+    s, cam = scenes.load_gpu(device, desc)
+    g = V.Guide(device, seed=1, batch_size=16384, steps_per_pass=4)
+    g.debug(analytic=True)
+    ctx = V.make_context(cam, s, spp=1, bounces=4, clamp=0.0, estimator=V.EST_GUIDED,
+                         rng=V.RNG_PCG, seed=0x77, guide=g, train=True)
+    img = np.zeros(W * H * 4, np.float32)
+    V.path_trace_tiles(ctx, V.ComputeTiles(W, H, 64, 64), img)
+    got = g.samples()
+    _, _, cand = _oracle_guided(desc, 1, 4, SPO_RNG_PCG, 0x77, sink=100000)
+    bits = lambda rows: sorted(  # noqa: E731
+        np.ascontiguousarray(r[3:13], np.float32).tobytes() for r in rows)
+    assert bits(got) == bits(cand)
+    g.close()
+    s.close()

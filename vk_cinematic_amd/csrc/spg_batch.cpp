@@ -226,7 +226,7 @@ int record(spg_Batch *b, hipStream_t st, const spg_TraceConfig &cfg,
                 HIPCHK(launch_guide_collect(st, p));
                 CHK(guide_train_pass(b->guide, st));
                 CHK(T1());
-                k += 3 + 7 * b->guide->cfg.stepsPerPass;
+                k += 3 + 4 * b->guide->cfg.stepsPerPass;
             }
             done += sp;
         }

@@ -4,7 +4,8 @@
 // k_guide_infer in spg_trace.hip; both use the MFMA blocks of spg_mlp.h.
 //
 // Training step over a batch of B samples (pn, n, v, wi, weight):
-//   k_guide_wsum    sum of the batch's weights (normalization to mean 1)
+//   k_guide_wsum    sum of the batch's weights (normalization to mean 1);
+//                   the step's loss at zero, the step count advanced
 //   k_guide_fwdbwd  per 64-sample tile: forward (keeping the ReLU masks),
 //                   d(-w log q)/d(outputs) per sample, backward through the
 //                   layers with the transposed weights; writes every
@@ -12,10 +13,10 @@
 //                   feature-major [64][B])
 //   k_guide_wgrad   dW_l = G_l H_l^T and db_l = G_l 1 as MFMA products with
 //                   the samples on K, one FP32 partial gradient per chunk
-//   k_guide_greduce the partials added in chunk order (the step's result
-//                   does not depend on scheduling)
-//   k_guide_adam    Adam on the FP32 master parameters, refreshes the FP16
-//                   forward and transposed copies, clears the gradient
+//   k_guide_adam    the partials added in chunk order (the step's result
+//                   does not depend on scheduling), Adam on the FP32 master
+//                   parameters, refreshes the FP16 forward and transposed
+//                   copies
 // Gradients carry a fixed loss scale (kLossScale) while in FP16 and are
 // clamped to the FP16 range; the FP32 accumulation is unscaled in Adam.
 #include "spg_internal.h"
@@ -114,9 +115,17 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_guide_eval(
 // Sum of the batch's weights in a fixed order (one block: each thread sums
 // a fixed stride of the batch, then a fixed tree), so a training step's
 // result does not depend on scheduling.
-__global__ __launch_bounds__(256) void k_guide_wsum(GuideTrainArgs a)
+//
+// Also begins a training step (`step` given): the loss starts at zero and the
+// step count advances.
+__global__ __launch_bounds__(256) void k_guide_wsum(GuideTrainArgs a, uint32_t *step)
 {
     __shared__ float part[256];
+    if (step && threadIdx.x == 0)
+    {
+        *a.loss = 0.0f;
+        *step += 1u;
+    }
     const uint32_t n = batch_count(a);
     float s = 0.0f;
     for (uint32_t j = threadIdx.x; j < n; j += 256)
@@ -354,20 +363,27 @@ __global__ __launch_bounds__(64) void k_guide_wgrad(GuideTrainArgs a)
     else wgrad_chunk<3>(a, l, k0, k1);
 }
 
-// The gradient: the chunks' partial gradients added in chunk order.
+// The chunks' partial gradients of parameter k added in chunk order.
+__device__ __forceinline__ float chunk_sum(const GuideTrainArgs &a, uint32_t n, uint32_t k)
+{
+    const uint32_t nPad = (n + 63) / 64 * 64;
+    const uint32_t chunks = (nPad + kGradChunk - 1) / kGradChunk;
+    float g = 0.0f;
+#pragma unroll 8
+    for (uint32_t c = 0; c < chunks; ++c) g += a.part[(size_t)c * kGParams + k];
+    return g;
+}
+
+// The gradient on its own (spg_guide_gradient).
 __global__ __launch_bounds__(256) void k_guide_greduce(GuideTrainArgs a)
 {
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
     if (k >= (uint32_t)kGParams) return;
-    const uint32_t nPad = (batch_count(a) + 63) / 64 * 64;
-    const uint32_t chunks = (nPad + kGradChunk - 1) / kGradChunk;
-    float g = 0.0f;
-    for (uint32_t c = 0; c < chunks; ++c) g += a.part[(size_t)c * kGParams + k];
-    a.grad[k] = g;
+    a.grad[k] = chunk_sum(a, batch_count(a), k);
 }
 
-// Adam on the master parameters, then the FP16 forward / transposed copies
-// and the FP32 biases; clears the gradient.  gradScale = 1 / (n * loss
+// The gradient's sum and Adam on the master parameters, then the FP16
+// forward / transposed copies and the FP32 biases.  gradScale = 1 / (n * loss
 // scale) is applied here (n read from the device).
 __global__ __launch_bounds__(256) void k_guide_adam(GuideTrainArgs a, GuideAdam h)
 {
@@ -381,7 +397,7 @@ __global__ __launch_bounds__(256) void k_guide_adam(GuideTrainArgs a, GuideAdam 
         const double t = (double)*h.step;
         const float c1 = (float)(1.0 - pow((double)h.beta1, t));
         const float c2 = (float)(1.0 - pow((double)h.beta2, t));
-        float gr = a.grad[k] * (1.0f / ((float)n * kLossScale));
+        float gr = chunk_sum(a, n, k) * (1.0f / ((float)n * kLossScale));
         float m = h.beta1 * a.m[k] + (1.0f - h.beta1) * gr;
         float v = h.beta2 * a.v[k] + (1.0f - h.beta2) * gr * gr;
         a.m[k] = m;
@@ -389,7 +405,6 @@ __global__ __launch_bounds__(256) void k_guide_adam(GuideTrainArgs a, GuideAdam 
         p -= h.lr * (m / c1) / (sqrtf(v / c2) + h.eps);
         a.params[k] = p;
     }
-    a.grad[k] = 0.0f;
     write_param_copies(a, k, p);
 }
 
@@ -421,32 +436,38 @@ hipError_t launch_guide_convert(hipStream_t s, const GuideTrainArgs &a)
     return hipGetLastError();
 }
 
-hipError_t launch_guide_gradient(hipStream_t s, const GuideTrainArgs &a,
-                                 uint32_t cus)
+// Every layer's partial weight gradients of the batch.
+static void launch_partials(hipStream_t s, const GuideTrainArgs &a, uint32_t cus)
 {
-    if (a.wsum) hipLaunchKernelGGL(k_guide_wsum, dim3(1), dim3(256), 0, s, a);
     uint32_t tiles = (a.batch + 63) / 64;
     uint32_t blocks = (tiles + kTrainWaves - 1) / kTrainWaves;
     if (blocks > cus) blocks = cus;
     hipLaunchKernelGGL(k_guide_fwdbwd, dim3(blocks), dim3(64 * kTrainWaves), 0, s, a);
     uint32_t chunks = (a.batch + kGradChunk - 1) / kGradChunk;
     hipLaunchKernelGGL(k_guide_wgrad, dim3(chunks, kGLayers), dim3(64), 0, s, a);
+}
+
+hipError_t launch_guide_gradient(hipStream_t s, const GuideTrainArgs &a,
+                                 uint32_t cus)
+{
+    if (a.wsum)
+        hipLaunchKernelGGL(k_guide_wsum, dim3(1), dim3(256), 0, s, a, (uint32_t *)nullptr);
+    launch_partials(s, a, cus);
     hipLaunchKernelGGL(k_guide_greduce, dim3((kGParams + 255) / 256), dim3(256), 0, s,
                        a);
     return hipGetLastError();
 }
 
-__global__ void k_guide_step(uint32_t *step) { *step += 1u; }
-
-hipError_t launch_guide_step(hipStream_t s, uint32_t *step)
+// Four launches: each small one costs about 4.4 us, so the loss's clear and
+// the step count ride on the weight sum and the gradient's sum on the update
+// (seven launches before).  k_guide_fwdbwd, batch 16384: 19.7 -> 11 us with
+// the staging's loads in flight together; 2 or 1 waves per block instead of 4
+// wait longer for the staging (29.7 and 50 us before that change).
+hipError_t launch_guide_train_step(hipStream_t s, const GuideTrainArgs &a,
+                                   const GuideAdam &h, uint32_t cus)
 {
-    hipLaunchKernelGGL(k_guide_step, dim3(1), dim3(1), 0, s, step);
-    return hipGetLastError();
-}
-
-hipError_t launch_guide_adam(hipStream_t s, const GuideTrainArgs &a,
-                             const GuideAdam &h)
-{
+    hipLaunchKernelGGL(k_guide_wsum, dim3(1), dim3(256), 0, s, a, h.step);
+    launch_partials(s, a, cus);
     hipLaunchKernelGGL(k_guide_adam, dim3((kGParams + 255) / 256), dim3(256), 0, s,
                        a, h);
     return hipGetLastError();

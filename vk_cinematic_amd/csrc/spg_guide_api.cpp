@@ -139,7 +139,8 @@ int upload_samples(spg_Guide *g, const float *rows, uint32_t n)
     return SPG_OK;
 }
 
-int adam_step(spg_Guide *g, const GuideTrainArgs &a, hipStream_t st)
+// One training step on `a` (its weights normalized).
+int train_step(spg_Guide *g, const GuideTrainArgs &a, hipStream_t st, uint32_t cus)
 {
     GuideAdam h{};
     h.lr = g->cfg.learningRate;
@@ -148,8 +149,7 @@ int adam_step(spg_Guide *g, const GuideTrainArgs &a, hipStream_t st)
     h.eps = kAdamEps;
     h.step = g->stepDev;
     h.apply = 1;
-    HIPCHK(launch_guide_step(st, g->stepDev));
-    HIPCHK(launch_guide_adam(st, a, h));
+    HIPCHK(launch_guide_train_step(st, a, h, cus));
     return SPG_OK;
 }
 
@@ -341,9 +341,7 @@ int guide_train_pass(spg_Guide *g, hipStream_t st)
     for (uint32_t k = 0; k < g->cfg.stepsPerPass; ++k)
     {
         GuideTrainArgs a = make_args(g, k * B, B, true, g->cfg.maxWeight);
-        HIPCHK(launch_clear_floats(st, g->loss, 1));
-        HIPCHK(launch_guide_gradient(st, a, cus));
-        CHK(adam_step(g, a, st));
+        CHK(train_step(g, a, st, cus));
     }
     return SPG_OK;
 }
@@ -539,9 +537,7 @@ int spg_guide_train(spg_Guide *g, const float *samples, uint32_t n, uint32_t ste
         uint32_t first = (k % batches) * B;
         lastN = std::min(B, n - first);
         GuideTrainArgs a = make_args(g, first, B, true, g->cfg.maxWeight);
-        HIPCHK(launch_clear_floats(d->stream, g->loss, 1));
-        HIPCHK(launch_guide_gradient(d->stream, a, cus));
-        CHK(adam_step(g, a, d->stream));
+        CHK(train_step(g, a, d->stream, cus));
     }
     float l = 0.0f;
     HIPCHK(hipMemcpyAsync(&l, g->loss, 4, hipMemcpyDeviceToHost, d->stream));

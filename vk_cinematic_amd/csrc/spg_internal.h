@@ -527,8 +527,8 @@ hipError_t launch_guide_eval(hipStream_t s, const _Float16 *w16, const float *bi
 hipError_t launch_guide_convert(hipStream_t s, const GuideTrainArgs &a);
 hipError_t launch_guide_gradient(hipStream_t s, const GuideTrainArgs &a,
                                  uint32_t cus);
-hipError_t launch_guide_adam(hipStream_t s, const GuideTrainArgs &a,
-                             const GuideAdam &h);
-// device Adam step count: += 1 before an update
-hipError_t launch_guide_step(hipStream_t s, uint32_t *step);
+// one training step: the loss restarted, the device step count advanced,
+// the gradient and the Adam update
+hipError_t launch_guide_train_step(hipStream_t s, const GuideTrainArgs &a,
+                                   const GuideAdam &h, uint32_t cus);
 }  // namespace spg
