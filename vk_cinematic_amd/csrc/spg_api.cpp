@@ -1287,6 +1287,7 @@ static int trace(const spg_Context *ctx, const spg_Tile *tiles, uint32_t count,
             int q = 0;
             for (uint32_t b = 0; b < cfg.bounces; ++b)
             {
+                p.bounce = b;
                 begin(kExtend);
                 HIPCHK(launch_extend(d->stream, p, q, d->persist));
                 // at the last bounce no hit scatters (a path at bounce b

@@ -188,6 +188,7 @@ int record(spg_Batch *b, hipStream_t st, const spg_TraceConfig &cfg,
             int q = 0;
             for (uint32_t bb = 0; bb < cfg.bounces; ++bb)
             {
+                p.bounce = bb;
                 CHK(T0(kExtend));
                 HIPCHK(launch_extend(st, p, q, ps));
                 CHK(T1());

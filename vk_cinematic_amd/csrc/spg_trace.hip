@@ -741,13 +741,6 @@ __global__ __launch_bounds__(256) void k_raygen(TraceParams p)
         p.paths.qpath[0][path] = path;
         p.paths.pathSlot[path] = slot;
         p.paths.pathSample[path] = sample;
-        p.paths.vcount[path] = 0;
-        p.paths.beta[path] = 1.0f;
-        p.paths.beta[cap + path] = 1.0f;
-        p.paths.beta[2 * cap + path] = 1.0f;
-        p.paths.radiance[path] = 0.0f;
-        p.paths.radiance[cap + path] = 0.0f;
-        p.paths.radiance[2 * cap + path] = 0.0f;
         store_rng(p, path, rng);
     }
 }
@@ -1018,6 +1011,15 @@ __device__ __forceinline__ float nee_hit_weight(const TraceParams &p, const DevS
 // One bounce of every queued path: surface, material, scatter, vertex record
 // (parity) or throughput update (unbiased), append continuing rays to queue
 // q^1 with a ballot + one atomic per wave.
+//
+// Bound by the latency of its reads (state, then the hit's triangle and
+// material) at the two waves per SIMD that the double-precision
+// transcendentals leave (182 registers; budgets for three to five waves spill:
+// a 1080p pass's 955 us become 924, 1172, 1438, the lamps' 602 become 653,
+// 704, 815).  So it moves only state that is read again: a path's vertex
+// count is the bounce, its throughput and radiance start from constants, and
+// a finished path keeps no throughput, stream or (unbiased) count (1080p room,
+// 6 bounces, 955 -> 843 us).
 template <bool kDouble, int kEst, bool kBatch>
 __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
 {
@@ -1046,7 +1048,7 @@ __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
             v3 d{p.paths.qd[q][i], p.paths.qd[q][cap + i], p.paths.qd[q][2 * cap + i]};
             float t = p.paths.ht[i];
             uint32_t inst = p.paths.hinst[i];
-            uint32_t vc = p.paths.vcount[path];
+            const uint32_t vc = p.bounce;  // a ray of bounce b has b vertices
             v3 V = -d;
             bool hit = inst != SPG_MISS && t > 0.0f;
             if (kEst == SPG_EST_PARITY)
@@ -1103,14 +1105,18 @@ __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
                 vt[4 * cap] = X.y;
                 vt[5 * cap] = X.z;
                 vt[6 * cap] = cosine;
-                p.paths.vcount[path] = vc + 1;
+                if (!push) p.paths.vcount[path] = vc + 1;
             }
             else if (kEst == SPG_EST_UNBIASED || kEst == SPG_EST_NEE)
             {
-                v3 beta{p.paths.beta[path], p.paths.beta[cap + path],
-                        p.paths.beta[2 * cap + path]};
-                v3 L{p.paths.radiance[path], p.paths.radiance[cap + path],
-                     p.paths.radiance[2 * cap + path]};
+                v3 beta{1.0f, 1.0f, 1.0f}, L{0.0f, 0.0f, 0.0f};
+                if (vc > 0)
+                {
+                    beta = v3{p.paths.beta[path], p.paths.beta[cap + path],
+                              p.paths.beta[2 * cap + path]};
+                    L = v3{p.paths.radiance[path], p.paths.radiance[cap + path],
+                           p.paths.radiance[2 * cap + path]};
+                }
                 if (hit)
                 {
                     hits++;
@@ -1187,13 +1193,15 @@ __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
                     else
                         L = L + had(beta, m.emission);
                 }
-                p.paths.beta[path] = beta.x;
-                p.paths.beta[cap + path] = beta.y;
-                p.paths.beta[2 * cap + path] = beta.z;
+                if (push)
+                {
+                    p.paths.beta[path] = beta.x;
+                    p.paths.beta[cap + path] = beta.y;
+                    p.paths.beta[2 * cap + path] = beta.z;
+                }
                 p.paths.radiance[path] = L.x;
                 p.paths.radiance[cap + path] = L.y;
                 p.paths.radiance[2 * cap + path] = L.z;
-                p.paths.vcount[path] = vc + 1;
             }
             else
             {
@@ -1308,9 +1316,11 @@ __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
                 vt[4 * cap] = X.y;
                 vt[5 * cap] = X.z;
                 vt[6 * cap] = c;
-                p.paths.vcount[path] = vc + 1;
+                if (!push) p.paths.vcount[path] = vc + 1;
             }
-            store_rng(p, path, rng);
+            // (the xorshift stream of a finished path goes on in the pixel's
+            // next sample)
+            if (push || !rng.pcg) store_rng(p, path, rng);
         }
         // compaction of continuing rays into queue nq (and of shadow rays
         // into queue 2): one atomic per block and queue
@@ -1378,7 +1388,7 @@ __global__ __launch_bounds__(256) void k_resolve_shadow(TraceParams p)
         // the vertex that took the light sample (the last one written)
         float *acc = p.paths.radiance + path;
         if (p.estimator == SPG_EST_GUIDED_NEE)
-            acc = p.paths.vtx + (size_t)(p.paths.vcount[path] - 1u) * 7 * cap + path;
+            acc = p.paths.vtx + (size_t)p.bounce * 7 * cap + path;
         acc[0] = acc[0] + C.x;
         acc[cap] = acc[cap] + C.y;
         acc[2 * cap] = acc[2 * cap] + C.z;
@@ -1645,7 +1655,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_guide_infer(TraceParams p,
             uint32_t inst = p.paths.hinst[i];
             float t = p.paths.ht[i];
             uint32_t path = p.paths.qpath[q][i];
-            if (inst != SPG_MISS && t > 0.0f && p.paths.vcount[path] + 1 < p.bounces)
+            if (inst != SPG_MISS && t > 0.0f && p.bounce + 1 < p.bounces)
             {
                 valid = true;
                 v3 o{qo[i], qo[cap + i], qo[2 * cap + i]};
