@@ -46,3 +46,17 @@ def test_rejects_bad_arguments(device):
         device.create_irradiance_cubemap(img, 0, 4)
     with pytest.raises(V.SpgError):
         device.create_irradiance_cubemap(img, 4, 4, 10.0, 7)
+
+
+def test_buffer_reuse(device):
+    """Calls with growing, shrinking and (beyond 64 MB) not kept source sizes
+    on one device give the bits of a first call on a new one."""
+    rng = np.random.default_rng(5)
+    sizes = [(16, 8, 4), (64, 32, 7), (16, 8, 4), (2176, 2048, 2), (64, 32, 7)]
+    for w, h, face in sizes:
+        img = rng.exponential(1.0, (h, w, 4)).astype(np.float32)
+        got, _ = device.create_irradiance_cubemap(img, face, face, 10.0, V.TX_DOUBLE)
+        fresh = V.Device(0)
+        want, _ = fresh.create_irradiance_cubemap(img, face, face, 10.0, V.TX_DOUBLE)
+        fresh.close()
+        assert np.array_equal(_bits(got), _bits(want))

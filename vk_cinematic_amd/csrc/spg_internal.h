@@ -248,6 +248,7 @@ struct TraceParams
 };
 
 constexpr uint32_t kStamps = 512;
+constexpr size_t kEnvKeepBytes = 64u << 20;
 // What a trace call reports to the host (pinned memory, written by its last
 // launch): the metrics, the device time of that launch, the launch stamps.
 struct TraceReport
@@ -330,6 +331,8 @@ struct spg_Device
     void *pathsBlock = nullptr;
     void *hostStage = nullptr;   // host-pixel calls: the tiles' pixels in slot
     size_t hostStageBytes = 0;   // order (RGBA32F), pinned, written by the device
+    void *env = nullptr;         // irradiance cube maps: source, faces and grid
+    size_t envBytes = 0;         // (kept up to kEnvKeepBytes)
     spg::TraceReport *report = nullptr; // pinned, written by the device
     unsigned long long *stamps = nullptr; // device, [kStamps]
     double clockKHz = 1e5;       // the device clock's rate
