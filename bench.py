@@ -51,14 +51,15 @@ BOX_BYTES, TRI_BYTES, ENTRY_BYTES = 24, 36, 128
 # x1.0 by the 1 GiB copy of `--workload copy` on the same box; config5: the
 # plain tracer's launches, `--no-guided`); the roofline's "traffic" is this
 # times the rays of one launch.
-TRAFFIC_BYTES_PER_RAY = {"config5": 1.5237e9 / 2036866, "soup": 1.0953e9 / 4194304}
+TRAFFIC_BYTES_PER_RAY = {"config5": 1.3923e9 / 2036866, "soup": 1.0627e9 / 4194304}
 # What bounds the closest-hit kernel in fact, from counter runs of the same
-# kernel and workload: the VALU issue rate, not HBM.  valu_busy: share of
-# the SIMDs' cycles issuing VALU work (SQ_INSTS_VALU x 4 cycles per wave64
+# kernel and workload: the VALU issue rate and the texture path, not HBM.
+# valu_busy: share of the SIMDs' cycles issuing VALU work (SQ_INSTS_VALU x 4 cycles per wave64
 # instruction over 1024 SIMDs x the dispatches' mean duration x 2.4 GHz);
 # valu_insts_per_ray: SQ_INSTS_VALU per traced ray.  The roofline "frac"
 # prices the algorithmic bytes, "traffic_frac" the counter-measured ones.
-LIMITER = {"config5": {"kind": "VALU issue", "valu_busy": 0.85, "valu_insts_per_ray": 253,
+LIMITER = {"config5": {"kind": "VALU issue and fetches", "valu_busy": 0.74,
+                       "valu_insts_per_ray": 172,
                        "source": "profiles/hbm_traffic_config5_soup.md"}}
 TRAFFIC_SOURCE = ("rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of the same kernel and "
                   "workload (profiles/hbm_traffic_config5_soup.md), FETCH x2.0 and "
@@ -1117,7 +1118,7 @@ def bench_post(args, V, scenes):
         "value": n / (t_acc + t_tm) / 1e6,
         "unit": "Mpixels/s",
         "ms_per_step": (t_acc + t_tm) * 1e3,
-        "dtype": "f32 -> u8 (f64 pow)" if tx == V.TX_DOUBLE else "f32 -> u8",
+        "dtype": "f32 -> u8 (bytes of the f64 pow)" if tx == V.TX_DOUBLE else "f32 -> u8",
         "config": {"workload": "post step on 1920x1080 RGBA32F: running mean of two "
                                "images, then Reinhard + gamma 1/2.2 to RGBA8"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,

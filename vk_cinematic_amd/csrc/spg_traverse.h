@@ -8,8 +8,8 @@
 // BVH) or leaving one after a hit (its model transform, for the world-space
 // t).  The walk is bound by vector instruction issue, and a wave pays for a
 // kind's instructions whether one of its lanes or all 64 are of that kind:
-// with every kind run in every iteration the 4M-triangle box scene took 253
-// instructions per ray and wave at 22% of the lanes busy.  So an iteration
+// with every kind run in every iteration the 4M-triangle room took 253
+// instructions per ray at 22% of the lanes busy (now 172).  So an iteration
 // runs ONE kind, the one that most lanes wait for (persistent_walk), and
 // the other lanes keep their state; what a lane does, and in which order,
 // does not depend on it.  A hit leaf child becomes the lane's leaf range
@@ -22,8 +22,8 @@
 // (sp_RayIntersectScene, src/sp_scene.cpp:263-276) and the mesh walk
 // continues on the same stack.
 //
-// Measured against all kinds per iteration, per pass: 4M-triangle box scene
-// at 512x512 2397 -> 1757 us, 2.5M-triangle room at 1080p 5443 -> 4415,
+// Measured against all kinds per iteration, per pass: 1M-triangle box scene
+// at 512x512 2397 -> 1757 us, 4M-triangle room at 1080p 5443 -> 4415,
 // eight-lamp scene with shadow rays 3979 -> 2784, 256x256 frame 361 -> 200,
 // 64x64 tile 110 -> 74; mesh rays: 2^21 on 500k triangles 664 -> 516.
 //
