@@ -1014,9 +1014,10 @@ __device__ __forceinline__ float nee_hit_weight(const TraceParams &p, const DevS
 //
 // Bound by the latency of its reads (state, then the hit's triangle and
 // material) at the two waves per SIMD that the double-precision
-// transcendentals leave (182 registers; budgets for three to five waves spill:
-// a 1080p pass's 955 us become 924, 1172, 1438, the lamps' 602 become 653,
-// 704, 815).  So it moves only state that is read again: a path's vertex
+// transcendentals leave (182 registers; budgets for three to five waves
+// spill: a 1080p pass's 955 us become 924, 1172, 1438, next-event
+// estimation's 602 become 653, 704, 815).  So it moves only state that is
+// read again: a path's vertex
 // count is the bounce, its throughput and radiance start from constants, and
 // a finished path keeps no throughput, stream or (unbiased) count (1080p room,
 // 6 bounces, 955 -> 843 us).

@@ -24,7 +24,7 @@
 //
 // Measured against all kinds per iteration, per pass: 1M-triangle box scene
 // at 512x512 2397 -> 1757 us, 4M-triangle room at 1080p 5443 -> 4415,
-// eight-lamp scene with shadow rays 3979 -> 2784, 256x256 frame 361 -> 200,
+// 1M-triangle room with shadow rays 3979 -> 2784, 256x256 frame 361 -> 200,
 // 64x64 tile 110 -> 74; mesh rays: 2^21 on 500k triangles 664 -> 516.
 //
 // Stack: the top entries of each lane live in LDS (4 or 8 KB per wave);
@@ -39,9 +39,10 @@ namespace spg {
 
 // Rays a wave takes from the shared counter with one atomic, at most (a
 // short ray list is divided evenly among the waves): same-address atomics
-// serialize in L2, so 64 costs the mesh walk 44% at 2^21 rays (744 us
-// against 516), and the scene walk 1-3% (box 1771 -> 1757 us, eight lamps
-// 2861 -> 2784, room 4386 -> 4415).
+// serialize in L2, so the mesh walk at 2^21 rays takes 744 us with 64 (and 16
+// waves per CU) against 530 with 128 (and 12).  The scene walk is the same
+// within 3%: box 1771 -> 1757 us, room with shadow rays 2861 -> 2784, 1080p
+// room 4386 -> 4415.
 constexpr uint32_t kSceneChunk = 128, kMeshChunk = 128;
 // A wave refills its idle lanes once kRefill of them wait (or all do): each
 // refill stalls the wave on the new rays' loads and setup, so refilling one
