@@ -1,0 +1,51 @@
+"""How launches divide their work (vk_cinematic_amd/csrc/spg_launch.h), on the
+CPU: the header is compiled with the host compiler and driven over the edges
+of its ranges, above all counts near 2^32, which no GPU test can hold."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                    "vk_cinematic_amd", "csrc")
+
+
+def _run(tmp_path, body):
+    """Compiles `body` (statements of main; return 0 = passed) and runs it."""
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text('#include "spg_launch.h"\n#include <stdio.h>\nusing namespace spg;\n'
+                   'int main()\n{\n' + body + '\n    return 0;\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-D__host__=", "-D__device__=",
+                    "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout
+    return r.stdout
+
+
+@pytest.mark.parametrize("rays", [0, 1, 63, 64, 65, 255, 257, 16383, 16385, 2560 * 128 + 1,
+                                  2**32 - 129, 2**32 - 128, 2**32 - 127, 2**32 - 64,
+                                  2**32 - 1])
+@pytest.mark.parametrize("waves", [1, 8, 2560, 8192])
+def test_chunks_cover_the_rays_once(tmp_path, rays, waves):
+    """The chunks are non-empty, follow one another and end at the last ray;
+    none is larger than the limit (in 64 bits, so that a wrapped end shows)."""
+    _run(tmp_path, f"""
+    const uint64_t n = {rays}ull;
+    const uint32_t want = walk_waves((uint32_t)n), grid = {waves}u;
+    const WorkChunks w((uint32_t)n, want < grid ? want : grid, 128u);
+    uint64_t at = 0;
+    for (uint32_t j = 0; j < w.chunks; ++j)
+    {{
+        const uint64_t lo = w.begin(j), hi = w.end(j);
+        if (lo != at || hi <= lo || hi > n || hi - lo > 128)
+        {{
+            printf("chunk %u of %u: [%llu, %llu) after %llu\\n", j, w.chunks,
+                   (unsigned long long)lo, (unsigned long long)hi, (unsigned long long)at);
+            return 1;
+        }}
+        at = hi;
+    }}
+    if (at != n) {{ printf("ends at %llu\\n", (unsigned long long)at); return 1; }}""")

@@ -18,6 +18,7 @@
 #include "spg_bvh.h"
 #include "spg_error.h"
 #include "spg_guide.h"
+#include "spg_launch.h"
 #include "spg_math.h"
 
 namespace spg {
@@ -35,19 +36,6 @@ constexpr int kTraceBlock = 64;  // traversal blocks are one wave
 // Resident waves per CU a persistent traversal launch may use (sizes the
 // global spill area of the traversal stacks).
 constexpr uint32_t kMaxPersistWavesPerCU = 32;
-
-// Waves that walk n rays (before the cap by occupancy): one per 64 rays, and
-// below 256 * 64 rays up to 256 waves with fewer rays each, one wave per CU
-// (a wave's time is that of its longest chain of steps, and lanes that wait
-// for other kinds of steps lengthen it).  96 or 128 rays per wave: the
-// 256x256 frame's walk takes 228 and 240 us instead of 200; 48 rays and at
-// least 512 waves: 214; 80 rays: 230.
-__host__ __device__ inline uint32_t walk_waves(uint32_t n)
-{
-    const uint32_t full = n / 64u + (n % 64u != 0u ? 1u : 0u);
-    const uint32_t few = n < 256u ? n : 256u;
-    return full > few ? full : few ? few : 1u;
-}
 
 // Per-launch work counter and stack spill area of persistent launches.
 struct Persist

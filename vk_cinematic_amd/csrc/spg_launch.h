@@ -1,0 +1,44 @@
+// How launches divide their work: plain arithmetic shared by the kernels,
+// the launch code and the CPU tests (which compile this header with the host
+// compiler), so it includes nothing of HIP.
+#pragma once
+
+#include <stdint.h>
+
+namespace spg {
+
+// Waves that walk n rays (before the cap by occupancy): one per 64 rays, and
+// below 256 * 64 rays up to 256 waves with fewer rays each, one wave per CU
+// (a wave's time is that of its longest chain of steps, and lanes that wait
+// for other kinds of steps lengthen it).  96 or 128 rays per wave: the
+// 256x256 frame's walk takes 228 and 240 us instead of 200; 48 rays and at
+// least 512 waves: 214; 80 rays: 230.
+__host__ __device__ inline uint32_t walk_waves(uint32_t n)
+{
+    const uint32_t full = n / 64u + (n % 64u != 0u ? 1u : 0u);
+    const uint32_t few = n < 256u ? n : 256u;
+    return full > few ? full : few ? few : 1u;
+}
+
+// The chunks of a list of n rays for `waves` waves: chunk j holds rays
+// [begin(j), end(j)).  An even share of the list, at most maxChunk rays.  No
+// sum here passes n, so none wraps for any 32-bit n.
+struct WorkChunks
+{
+    uint32_t n, chunk, chunks;
+    __host__ __device__ inline WorkChunks(uint32_t rays, uint32_t waves, uint32_t maxChunk)
+        : n(rays)
+    {
+        const uint32_t last = n ? n - 1u : 0u, share = last / waves + 1u;
+        chunk = share < maxChunk ? share : maxChunk;
+        chunks = n ? last / chunk + 1u : 0u;
+    }
+    __host__ __device__ inline uint32_t begin(uint32_t j) const { return j * chunk; }
+    __host__ __device__ inline uint32_t end(uint32_t j) const
+    {
+        const uint32_t lo = j * chunk, left = n - lo;
+        return lo + (chunk < left ? chunk : left);
+    }
+};
+
+}  // namespace spg

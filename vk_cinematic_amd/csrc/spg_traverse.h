@@ -586,24 +586,22 @@ __device__ __forceinline__ void trav_begin_mesh(const DevMesh &M, Trav &s, v3 o,
     s.cur = 0;
 }
 
-// The rays of a persistent launch in chunks, handed to its waves: chunk j
-// holds rays [j * chunk, (j + 1) * chunk).  A wave's first chunk is the one
-// at its own position, the further ones come from the counter (zero on
-// entry), so a launch whose rays fit its waves makes no atomic at all and in
-// the others no wave starts by waiting for one (same-address atomics take
-// 11 ns each: 56 us for 5120 waves that start together).
+// The rays of a persistent launch in chunks, handed to its waves.  A wave's
+// first chunk is the one at its own position, the further ones come from the
+// counter (zero on entry), so a launch whose rays fit its waves makes no
+// atomic at all and in the others no wave starts by waiting for one
+// (same-address atomics take 11 ns each: 56 us for 5120 waves that start
+// together).
 struct WorkSource
 {
     uint32_t *counter;
-    uint32_t n, waves, chunk, chunks;
+    uint32_t waves;
+    WorkChunks work;
     bool first;
     __device__ __forceinline__ WorkSource(uint32_t *c, uint32_t rays, uint32_t w,
                                           uint32_t maxChunk)
-        : counter(c), n(rays), waves(w), first(true)
+        : counter(c), waves(w), work(rays, w, maxChunk), first(true)
     {
-        const uint32_t last = n ? n - 1u : 0u;  // (n + waves - 1 could wrap)
-        chunk = min(last / waves + 1u, maxChunk);
-        chunks = n ? last / chunk + 1u : 0u;
     }
     // The wave's next chunk as rays [lo, hi); false: none left (every
     // further call says so too).  Wave-uniform.
@@ -613,16 +611,16 @@ struct WorkSource
         if (!first)
         {
             uint32_t k = 0;
-            if (waves < chunks && lane == 0) k = atomicAdd(counter, 1u);
+            if (waves < work.chunks && lane == 0) k = atomicAdd(counter, 1u);
             // wave-uniform (a scalar register), so the loop's exit is
             // uniform and the compiler keeps no per-lane copies of the
             // lane state across it
             j = waves + __builtin_amdgcn_readfirstlane(k);
         }
         first = false;
-        const bool some = j < chunks;
-        lo = some ? j * chunk : 0u;
-        hi = some ? min(n, lo + chunk) : 0u;
+        const bool some = j < work.chunks;
+        lo = some ? work.begin(j) : 0u;
+        hi = some ? work.end(j) : 0u;
         return some;
     }
 };
