@@ -49,3 +49,32 @@ def test_chunks_cover_the_rays_once(tmp_path, rays, waves):
         at = hi;
     }}
     if (at != n) {{ printf("ends at %llu\\n", (unsigned long long)at); return 1; }}""")
+
+
+@pytest.mark.parametrize("most", [2048, 65535])   # tone map; accumulation
+@pytest.mark.parametrize("items", [1, 255, 256, 257, 2048 * 256 + 3, 2**32 - 65535 * 256,
+                                   2**32 - 2048 * 256 + 1, 2**32 - 256, 2**32 - 1])
+def test_strided_loops_end_and_cover_the_items_once(tmp_path, items, most):
+    """The grid has a block for every 256 items up to the limit, and threads
+    at both ends of it (and where the count's remainder falls) step through
+    their own residue once and stop."""
+    _run(tmp_path, f"""
+    const uint64_t n = {items}ull;
+    const uint32_t grid = stride_blocks((uint32_t)n, 256, {most}u);
+    const uint64_t want = (n + 255) / 256 < {most}ull ? (n + 255) / 256 : {most}ull;
+    if (grid != want) {{ printf("grid %u\\n", grid); return 1; }}
+    const uint64_t step = grid * 256ull;
+    const uint64_t at[] = {{0, 1, step / 2, n % step, (n + step - 1) % step, step - 1}};
+    for (uint64_t first : at)
+    {{
+        uint64_t expect = first;
+        for (uint32_t i = (uint32_t)first; i < (uint32_t)n;
+             i = stride_next(i, (uint32_t)step, (uint32_t)n), expect += step)
+            if (i != expect)
+            {{
+                printf("thread %llu: item %u after %llu\\n", (unsigned long long)first, i,
+                       (unsigned long long)(expect - step));
+                return 1;
+            }}
+        if (expect < n) {{ printf("thread %llu ends early\\n", (unsigned long long)first); return 1; }}
+    }}""")

@@ -41,4 +41,18 @@ struct WorkChunks
     }
 };
 
+// A grid-stride loop's next index, n at its end: `i + step` would wrap where n
+// is within a step of 2^32, and the thread would start over for ever.
+__host__ __device__ inline uint32_t stride_next(uint32_t i, uint32_t step, uint32_t n)
+{
+    return n - i > step ? i + step : n;
+}
+
+// Blocks of `block` threads for n items, at most `most`.
+__host__ __device__ inline uint32_t stride_blocks(uint32_t n, uint32_t block, uint32_t most)
+{
+    const uint32_t need = n / block + (n % block != 0u ? 1u : 0u);
+    return need < most ? need : most;
+}
+
 }  // namespace spg

@@ -12,7 +12,7 @@ __global__ __launch_bounds__(256) void k_accumulate(float4 *__restrict__ dst,
                                                     float added, float total)
 {
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < pixels;
-         i += gridDim.x * 256)
+         i = stride_next(i, gridDim.x * 256, pixels))
     {
         float4 a = dst[i], b = src[i];
         a.x = (a.x * before + b.x * added) / total;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void k_tonemap(const float4 *__restrict__ src,
         __syncthreads();
     }
     for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < pixels;
-         i += gridDim.x * 256)
+         i = stride_next(i, gridDim.x * 256, pixels))
     {
         const float4 c = src[i];
         const float ch[3] = {c.x, c.y, c.z};
@@ -127,7 +127,7 @@ hipError_t launch_accumulate(hipStream_t s, float4 *dst, const float4 *src,
                              uint32_t pixels, uint32_t before, uint32_t added)
 {
     if (pixels == 0) return hipSuccess;
-    const uint32_t blocks = (pixels + 255) / 256 < 65535u ? (pixels + 255) / 256 : 65535u;
+    const uint32_t blocks = stride_blocks(pixels, 256, 65535u);
     k_accumulate<<<blocks, 256, 0, s>>>(dst, src, pixels, (float)before, (float)added,
                                         (float)before + (float)added);
     return hipGetLastError();
@@ -138,8 +138,7 @@ hipError_t launch_tonemap(hipStream_t s, const float4 *src, uint32_t pixels,
 {
     if (pixels == 0) return hipSuccess;
     const uint32_t most = dbl ? 2048u : 65535u;
-    const uint32_t blocks = pixels / 256u + (pixels % 256u ? 1u : 0u);
-    const uint32_t grid = blocks < most ? blocks : most;
+    const uint32_t grid = stride_blocks(pixels, 256, most);
     if (dbl) k_tonemap<true><<<grid, 256, 0, s>>>(src, pixels, exposure, out);
     else k_tonemap<false><<<grid, 256, 0, s>>>(src, pixels, exposure, out);
     return hipGetLastError();
