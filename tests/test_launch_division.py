@@ -78,3 +78,15 @@ def test_strided_loops_end_and_cover_the_items_once(tmp_path, items, most):
             }}
         if (expect < n) {{ printf("thread %llu ends early\\n", (unsigned long long)first); return 1; }}
     }}""")
+
+
+def test_tuned_refill_thresholds_differ_from_the_default(tmp_path):
+    """Every threshold the batch tuner times is another launch than the
+    default (0 stands for it): valid, distinct and not the default's value."""
+    _run(tmp_path, """
+    for (uint32_t a : kRefillSweep)
+    {
+        int same = a == kSceneRefill ? 1 : 0;
+        for (uint32_t b : kRefillSweep) same += a == b ? 1 : 0;
+        if (a < 1 || a > 64 || same != 1) { printf("threshold %u\\n", a); return 1; }
+    }""")

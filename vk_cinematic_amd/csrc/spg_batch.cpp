@@ -283,7 +283,8 @@ std::map<std::string, TunedShape> gTuned;
 // Candidates: wavefront capacity x resident traversal blocks, each timed on
 // one sample per pixel of the whole batch, then the traversal's refill
 // threshold (idle lanes a wave waits for before taking new rays) at the
-// fastest of those; the fastest is kept, and remembered for the key.
+// fastest of those; the fastest (by more than the timings' spread, else the
+// earlier candidate) is kept, and remembered for the key.
 int autotune(spg_Batch *b, uint32_t cus, const std::string &key)
 {
     spg_TraceConfig one = b->cfg;
@@ -312,7 +313,7 @@ int autotune(spg_Batch *b, uint32_t cus, const std::string &key)
             b->maxBlocks = mb;
             CHK(timed(b, one, &ms));
             ++tried;
-            if (tried == 1 || ms < best)
+            if (tried == 1 || tuned_better(ms, best))
             {
                 best = ms;
                 bestCap = c;
@@ -322,12 +323,12 @@ int autotune(spg_Batch *b, uint32_t cus, const std::string &key)
     }
     CHK(alloc_state(b, bestCap));
     b->maxBlocks = bestBlocks;
-    for (uint32_t rf : {32u, 48u})
+    for (uint32_t rf : kRefillSweep)
     {
         b->refill = rf;
         CHK(timed(b, one, &ms));
         ++tried;
-        if (ms < best)
+        if (tuned_better(ms, best))
         {
             best = ms;
             bestRefill = rf;

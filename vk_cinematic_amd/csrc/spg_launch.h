@@ -41,6 +41,23 @@ struct WorkChunks
     }
 };
 
+// A wave refills its idle lanes once kRefill of them wait (or all do): each
+// refill stalls the wave on the new rays' loads and setup, so refilling one
+// lane per iteration adds a memory round trip to nearly every step, while
+// waiting for all 64 leaves the wave running its longest ray alone.  Scene
+// walk: 40 instead of 32 costs 2-3% (box 1820 against 1771 us, room 4532
+// against 4386); mesh walk: 48 instead of 32 costs 2% (527 against 516 us).
+constexpr uint32_t kSceneRefill = 32, kMeshRefill = 32;
+// Refill thresholds of the scene walk that a batch's tuner times against the
+// default (24 grid scenes at 2^22 paths in flight: 5.06 ms per sample with
+// 32, 4.92 with 40, 5.05 with 48; eight grid scenes of 64 to 512 pixels a
+// side at 2^20: 1.13, 1.14, 1.16).
+constexpr uint32_t kRefillSweep[] = {40, 48};
+// A candidate of the tuner replaces the best so far only where its time is
+// shorter by more than 2%: timings of one shape differ by 1-4% from run to
+// run.
+inline bool tuned_better(float ms, float best) { return ms < 0.98f * best; }
+
 // A grid-stride loop's next index, n at its end: `i + step` would wrap where n
 // is within a step of 2^32, and the thread would start over for ever.
 __host__ __device__ inline uint32_t stride_next(uint32_t i, uint32_t step, uint32_t n)

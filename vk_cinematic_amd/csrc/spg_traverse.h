@@ -44,13 +44,6 @@ namespace spg {
 // within 3%: box 1771 -> 1757 us, room with shadow rays 2861 -> 2784, 1080p
 // room 4386 -> 4415.
 constexpr uint32_t kSceneChunk = 128, kMeshChunk = 128;
-// A wave refills its idle lanes once kRefill of them wait (or all do): each
-// refill stalls the wave on the new rays' loads and setup, so refilling one
-// lane per iteration adds a memory round trip to nearly every step, while
-// waiting for all 64 leaves the wave running its longest ray alone.  Scene
-// walk: 40 instead of 32 costs 2-3% (box 1820 against 1771 us, room 4532
-// against 4386); mesh walk: 48 instead of 32 costs 2% (527 against 516 us).
-constexpr uint32_t kSceneRefill = 32, kMeshRefill = 32;
 // The top kShort entries of each lane's stack live in LDS (kShort * 256
 // bytes per wave), deeper ones spill to global memory: 40 for the scene walk
 // costs the room 4% (4539 us against 4359), 80 for the mesh walk gains
