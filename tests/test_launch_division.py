@@ -90,3 +90,15 @@ def test_tuned_refill_thresholds_differ_from_the_default(tmp_path):
         for (uint32_t b : kRefillSweep) same += a == b ? 1 : 0;
         if (a < 1 || a > 64 || same != 1) { printf("threshold %u\\n", a); return 1; }
     }""")
+
+
+def test_spill_area_begins_where_the_shortest_lds_stack_ends(tmp_path):
+    """Entry i of a walk's stack spills at row i - kMinShortStack at the
+    lowest: no row below the first one used, none used below the first."""
+    _run(tmp_path, """
+    const int shortest = kSceneShortStack < kMeshShortStack ? kSceneShortStack : kMeshShortStack;
+    if (kMinShortStack != shortest)
+    {
+        printf("area from entry %d, stacks spill from %d\\n", kMinShortStack, shortest);
+        return 1;
+    }""")

@@ -48,6 +48,16 @@ struct WorkChunks
 // walk: 40 instead of 32 costs 2-3% (box 1820 against 1771 us, room 4532
 // against 4386); mesh walk: 48 instead of 32 costs 2% (527 against 516 us).
 constexpr uint32_t kSceneRefill = 32, kMeshRefill = 32;
+// The top kShort entries of each lane's stack live in LDS (kShort * 256
+// bytes per wave), deeper ones spill to global memory: 40 for the scene walk
+// costs the room 4% (4539 us against 4359), 80 for the mesh walk gains
+// nothing over 32.
+constexpr int kSceneShortStack = 16, kMeshShortStack = 32;
+// The spill area's first entry: what no walk keeps in LDS (2.1 MB per entry on
+// 256 CUs).
+constexpr int kMinShortStack =
+    kSceneShortStack < kMeshShortStack ? kSceneShortStack : kMeshShortStack;
+
 // Refill thresholds of the scene walk that a batch's tuner times against the
 // default (24 grid scenes at 2^22 paths in flight: 5.06 ms per sample with
 // 32, 4.92 with 40, 5.05 with 48; eight grid scenes of 64 to 512 pixels a

@@ -44,12 +44,6 @@ namespace spg {
 // within 3%: box 1771 -> 1757 us, room with shadow rays 2861 -> 2784, 1080p
 // room 4386 -> 4415.
 constexpr uint32_t kSceneChunk = 128, kMeshChunk = 128;
-// The top kShort entries of each lane's stack live in LDS (kShort * 256
-// bytes per wave), deeper ones spill to global memory: 40 for the scene walk
-// costs the room 4% (4539 us against 4359), 80 for the mesh walk gains
-// nothing over 32.
-constexpr int kSceneShortStack = 16, kMeshShortStack = 32;
-constexpr int kMinShortStack = 8;  // sizes the spill area
 // The weights of the step kinds when a wave chooses the kind to run: a lane
 // that waits for a rare kind costs as much as one that waits for a node, but
 // the node step is the longest (about 150 instructions against 60 to 90),
@@ -632,6 +626,7 @@ __device__ __forceinline__ void persistent_walk(SceneView &sv, uint32_t n,
                                                 Store store, Counts &cnt,
                                                 uint32_t &rays)
 {
+    static_assert(kShort >= kMinShortStack, "the spill area holds every deeper entry");
     const uint32_t want = walk_waves(n), waves = want < gridDim.x ? want : gridDim.x;
     if (blockIdx.x >= waves) return;
     __shared__ int lds[kShort * 64];
