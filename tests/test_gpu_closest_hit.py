@@ -186,3 +186,39 @@ def test_ray_counts_around_waves_and_chunks(device, n):
     bp, bt = _brute(tris, np.asarray(o).reshape(-1, 3), d)
     assert np.array_equal(prim, bp)
     assert np.array_equal(t.view(np.uint32), bt.view(np.uint32))
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_infinite_directions_over_overflowing_distances(device, axis):
+    """An infinite direction component has the finite inverse 0, and a node
+    whose distance from the origin overflows makes 0 times infinity of it:
+    such a ray takes the reference's compare-and-select box test (which misses
+    a box with a NaN on the z axis and ignores one on the others).  The
+    restatement of the walk decides with a finiteness test of every factor;
+    triangle, t and both test counts equal it."""
+    rng = np.random.default_rng(8)
+    n, m_tris = 3000, 2000
+    tris = rng.uniform(-1e32, 1e32, (m_tris, 1, 3)) + rng.uniform(-1e31, 1e31, (m_tris, 3, 3))
+    tris[:, :, axis] += 1.5e38
+    tris = np.ascontiguousarray(tris.reshape(m_tris, 9).astype(np.float32))
+    o = rng.uniform(-1e32, 1e32, (n, 3))
+    o[:, axis] = np.where(rng.random(n) < 0.5, -2.5e38, 0.0)
+    o = o.astype(np.float32)
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    d[:, axis] = np.where(rng.random(n) < 0.7, np.inf, 1.0)
+    s, m = _scene(device, tris)
+    bufs = [device.upload(np.ascontiguousarray(a[:, k])) for a in (o, d) for k in range(3)]
+    outp, outt = device.alloc(4 * n), device.alloc(4 * n)
+    st = V.TraversalStats()
+    V.check(V.lib().spg_intersect_closest_device(
+        s.handle, m, *[b.ptr for b in bufs], n, outp.ptr, outt.ptr, None, None,
+        C.byref(st)))
+    nodes, order, _ = s.wide_export(m)
+    tp, tt = np.zeros(n, np.uint32), np.zeros(n, np.float32)
+    box, tri = C.c_uint64(), C.c_uint64()
+    oracle().spo_wide_closest(np.ascontiguousarray(nodes.ravel()), order, tris.ravel(),
+                              np.ascontiguousarray(np.concatenate([o, d], 1).ravel()), n, 16,
+                              tp, tt, C.byref(box), C.byref(tri))
+    assert np.array_equal(outp.download(np.uint32, n), tp)
+    assert np.array_equal(outt.download(np.float32, n).view(np.uint32), tt.view(np.uint32))
+    assert (st.boxTests, st.triTests) == (box.value, tri.value)

@@ -379,11 +379,12 @@ __device__ __forceinline__ void step_node(const SceneView &sv, Trav &s,
         const float bx = (A.x - o.x) * inv.x, by = (A.y - o.y) * inv.y,
                     bz = (A.z - o.z) * inv.z;
         const float cx24 = ax * 16777216.0f, cy24 = ay * 16777216.0f, cz24 = az * 16777216.0f;
-        // finite factors (with a finite ray none can be NaN: |s|, |p - o| and
-        // |inv| are numbers, so a product is finite or infinite)
-        const float big =
-            fmaxf(fmaxf(fmaxf(fabsf(cx24), fabsf(cy24)), fmaxf(fabsf(cz24), fabsf(bx))),
-                  fmaxf(fabsf(by), fabsf(bz)));
+        // finite factors: the IEEE maximum keeps a NaN (v_maximum3; v_max3
+        // would drop it), which an infinite direction gives where p - o
+        // overflows, 0 times infinity
+        auto mx = [](float x, float y) { return __builtin_elementwise_maximum(x, y); };
+        const float big = mx(mx(mx(fabsf(cx24), fabsf(cy24)), mx(fabsf(cz24), fabsf(bx))),
+                             mx(fabsf(by), fabsf(bz)));
         const bool fast = s.mm && big < INFINITY;
         // per axis the near plane is the lo field where inv > 0 (a
         // positive a makes t increase with q) and the hi field where
