@@ -2,6 +2,8 @@
 bytes (double-evaluated pow), progressive accumulation of two trace calls
 equals the oracle's accumulation of the same two images and the single
 render of all their samples to FP32 rounding."""
+import math
+
 import numpy as np
 import pytest
 
@@ -54,14 +56,42 @@ def test_progressive_accumulation(device):
     s.close()
 
 
+def _around_steps():
+    """Radiances whose c / (1 + c), in float32 as the tone map forms it, lies
+    as closely below and above each of the 255 steps of the byte as a float32
+    c reaches (the step itself and the float below it wherever they have a c:
+    a value just below a power of two often has none), and the floats within
+    40 of each step's preimage."""
+    picked, tight = [], 0
+    for k in range(1, 256):
+        def byte(x):   # of the double power, rounded once to float
+            g = np.array([math.pow(float(v), float(np.float32(1.0) / np.float32(2.2)))
+                          for v in x]).astype(np.float32)
+            return np.rint(g * np.float32(255.0))
+
+        at = ((k - 0.5) / 255.0) ** 2.2
+        c0 = at / (1.0 - at)
+        width = int(60 + 8 * (1 + c0))   # about 1 + c floats c share a value
+        c = (np.float32(c0).view(np.int32) + np.arange(-width, width + 1)).astype(np.int32)
+        c = c.view(np.float32)
+        x = c / (np.float32(1.0) + c)
+        above = byte(x) >= k
+        assert above.any() and not above.all()
+        lo = int(np.argmax(np.where(above, -1.0, x)))    # (x need not rise with c:
+        hi = int(np.argmin(np.where(above, x, 2.0)))     # 1 + c rounds too)
+        tight += int(x[hi].view(np.int32) - x[lo].view(np.int32) == 1)
+        picked += [c[lo], c[hi]]
+        picked += list(c[width - 40: width + 41])
+    assert tight > 200                   # most steps have both neighbours
+    return np.array(picked, np.float32)
+
+
 @pytest.mark.parametrize("pixels", [1, 255, 257, 2048 * 256 + 3])
 def test_tonemap_bytes_at_every_step(device, pixels):
-    """Radiances around each of the 255 steps of the byte (the floats within
-    40 of the step's preimage c = x / (1 - x), x = ((k - 1/2) / 255)^2.2), and
-    the values outside [0, 1): the oracle's bytes exactly."""
-    x = ((np.arange(1, 256) - 0.5) / 255.0) ** 2.2
-    c = (x / (1.0 - x)).astype(np.float32).view(np.int32)
-    near = (c[:, None] + np.arange(-40, 41)).astype(np.int32).ravel().view(np.float32)
+    """Radiances around each of the 255 steps of the byte, and the values
+    outside [0, 1): the oracle's bytes exactly.  (The steps themselves are
+    pinned float by float on the CPU, tests/test_post.py.)"""
+    near = _around_steps()
     odd = np.array([0.0, -0.0, 1e-45, 1e-38, 3e38, np.inf, -np.inf, np.nan, -0.5, -1.0,
                     -2.0, -1e-45, -3e38, 2.0 ** 24, 2.0 ** 25, 1.0], np.float32)
     px = np.resize(np.concatenate([odd, near]), pixels * 4).astype(np.float32)

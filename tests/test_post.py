@@ -1,6 +1,10 @@
 """The step after the path: the oracle's tone mapping (PerformToneMapping,
 src/shaders/post_processing.frag.glsl:19-26) and progressive accumulation
 against closed forms, and the PFM writer (a host function of the library)."""
+import math
+import os
+import re
+
 import numpy as np
 import pytest
 
@@ -51,3 +55,24 @@ def test_pfm_round_trip(tmp_path):
     assert data[:len(head)] == head
     body = np.frombuffer(data[len(head):], "<f4").reshape(2, 3, 3)
     assert np.array_equal(body[::-1], img[:, :, :3])
+
+
+def test_tone_steps_are_the_steps_of_the_double_power():
+    """The tone map's table (read from the kernel's source): at entry k the
+    byte of the double-precision power, rounded once to float, is k, and at
+    the float below it k - 1, for all 255 steps; in between the power rises
+    with x, so the table is the whole function."""
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                        "vk_cinematic_amd", "csrc", "spg_post.hip")
+    body = re.search(r"kToneSteps\[256\] = \{(.*?)\};", open(path).read(), re.S).group(1)
+    steps = np.array([int(w, 16) for w in re.findall(r"0x[0-9A-Fa-f]{8}", body)], np.uint32)
+    assert steps.size == 256 and steps[0] == 0 and np.all(np.diff(steps.astype(np.int64)) > 0)
+
+    def byte(bits):
+        x = np.array([bits], np.uint32).view(np.float32)[0]
+        g = np.float32(math.pow(float(x), float(np.float32(1.0) / np.float32(2.2))))
+        return int(np.rint(g * np.float32(255.0)))
+
+    for k in range(1, 256):
+        assert (byte(steps[k] - 1), byte(steps[k])) == (k - 1, k), k
+    assert byte(0x3F800000) == 255   # x = 1
