@@ -391,7 +391,7 @@ __global__ __launch_bounds__(256) void k_guide_adam(GuideTrainArgs a, GuideAdam 
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
     if (k >= (uint32_t)kGParams) return;
     float p = a.params[k];
-    if (n > 0 && h.apply)
+    if (n > 0)
     {
         // bias corrections 1 - beta^t in double, rounded once
         const double t = (double)*h.step;

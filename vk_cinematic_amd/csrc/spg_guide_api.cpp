@@ -148,7 +148,6 @@ int train_step(spg_Guide *g, const GuideTrainArgs &a, hipStream_t st, uint32_t c
     h.beta2 = kBeta2;
     h.eps = kAdamEps;
     h.step = g->stepDev;
-    h.apply = 1;
     HIPCHK(launch_guide_train_step(st, a, h, cus));
     return SPG_OK;
 }
@@ -175,7 +174,6 @@ int set_params_locked(spg_Guide *g, const float *p)
                           hipMemcpyHostToDevice, d->stream));
     HIPCHK(hipMemsetAsync(g->m, 0, sizeof(float) * kGParams, d->stream));
     HIPCHK(hipMemsetAsync(g->v, 0, sizeof(float) * kGParams, d->stream));
-    HIPCHK(hipMemsetAsync(g->grad, 0, sizeof(float) * kGParams, d->stream));
     HIPCHK(launch_set_counter(d->stream, g->stepDev, 0u));
     HIPCHK(launch_guide_convert(d->stream, make_args(g, 0, 64, false, 0.0f)));
     HIPCHK(hipStreamSynchronize(d->stream));
@@ -511,7 +509,6 @@ int spg_guide_gradient(spg_Guide *g, const float *samples, uint32_t n, int norma
     HIPCHK(hipMemcpyAsync(grad, g->grad, sizeof(float) * kGParams,
                           hipMemcpyDeviceToHost, d->stream));
     HIPCHK(hipMemcpyAsync(&l, g->loss, 4, hipMemcpyDeviceToHost, d->stream));
-    HIPCHK(launch_clear_floats(d->stream, g->grad, kGParams));
     HIPCHK(hipStreamSynchronize(d->stream));
     const float scale = 1.0f / ((float)n * kLossScale);
     for (int k = 0; k < kGParams; ++k) grad[k] *= scale;
@@ -708,7 +705,6 @@ int spg_guide_load(spg_Guide *g, const char *path)
     for (int k = 0; k < 3; ++k)
         HIPCHK(hipMemcpyAsync(dst[k], st.data() + (size_t)k * kGParams,
                               sizeof(float) * kGParams, hipMemcpyHostToDevice, d->stream));
-    HIPCHK(launch_clear_floats(d->stream, g->grad, kGParams));
     HIPCHK(launch_set_counter(d->stream, g->stepDev, head[2]));
     HIPCHK(launch_guide_convert(d->stream, make_args(g, 0, 64, false, 0.0f)));
     HIPCHK(hipStreamSynchronize(d->stream));

@@ -204,7 +204,7 @@ struct TraceParams
     // writes its items' images)
     uint32_t firstPass, lastPass;
     float *image, *slotOut;
-    uint32_t bounce;             // of this k_guide_infer / k_shade / k_resolve_shadow
+    uint32_t bounce;             // of this k_shade / k_resolve_shadow
     uint32_t firstLaunch;        // the call's first pass: zero the metrics
     // launch start times (device clock), written at stamps[stamp] by the
     // launch's first block; stamp >= kStamps: not recorded
@@ -273,7 +273,6 @@ struct GuideAdam
 {
     float lr, beta1, beta2, eps;
     uint32_t *step;
-    uint32_t apply;
 };
 
 }  // namespace spg

@@ -1621,7 +1621,8 @@ __global__ __launch_bounds__(1024) void k_guide_emit(TraceParams p)
     }
 }
 
-// Guide inference for every queued ray that will scatter: hit surface ->
+// Guide inference for every queued ray that will scatter (every one that hit:
+// there is no launch for the last bounce): hit surface ->
 // encoding -> MLP (FP16 MFMA, FP32 accumulation) -> vMF mixture, stored
 // per queue entry for k_shade.  One block of kInferWaves waves per CU
 // shares the weights and biases in LDS (41,344 + 1,216 bytes); each wave
@@ -1656,7 +1657,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_guide_infer(TraceParams p,
             uint32_t inst = p.paths.hinst[i];
             float t = p.paths.ht[i];
             uint32_t path = p.paths.qpath[q][i];
-            if (inst != SPG_MISS && t > 0.0f && p.bounce + 1 < p.bounces)
+            if (inst != SPG_MISS && t > 0.0f)
             {
                 valid = true;
                 v3 o{qo[i], qo[cap + i], qo[2 * cap + i]};
