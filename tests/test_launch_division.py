@@ -102,3 +102,12 @@ def test_spill_area_begins_where_the_shortest_lds_stack_ends(tmp_path):
         printf("area from entry %d, stacks spill from %d\\n", kMinShortStack, shortest);
         return 1;
     }""")
+
+
+@pytest.mark.parametrize("words", [6, 7])   # a scene query's ray and its result
+def test_record_offsets_do_not_wrap(tmp_path, words):
+    """The last record below 2^32 words, the first above it and the last ray."""
+    _run(tmp_path, f"""
+    const uint64_t at[] = {{0, 1, 613566756, 613566757, 715827882, 715827883, 4294967295}};
+    for (uint64_t i : at)
+        if (record_at((uint32_t)i, {words}u) != i * {words}ull) return 1;""")

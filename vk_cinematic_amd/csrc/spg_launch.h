@@ -68,6 +68,13 @@ constexpr uint32_t kRefillSweep[] = {40, 48};
 // run.
 inline bool tuned_better(float ms, float best) { return ms < 0.98f * best; }
 
+// Where record i of a list of `words` words each begins (i * words passes 2^32
+// from 715,827,883 rays of 6 words on).
+__host__ __device__ inline uint64_t record_at(uint32_t i, uint32_t words)
+{
+    return (uint64_t)i * words;
+}
+
 // A grid-stride loop's next index, n at its end: `i + step` would wrap where n
 // is within a step of 2^32, and the thread would start over for ever.
 __host__ __device__ inline uint32_t stride_next(uint32_t i, uint32_t step, uint32_t n)

@@ -634,13 +634,13 @@ __global__ __launch_bounds__(kTraceBlock) void k_intersect_scene(
     uint32_t rays = 0;
     SceneView sv = scene_view(S);
     auto begin = [&](uint32_t i, Trav &s) {
-        trav_begin_scene(sv, s, v3{rays6[6 * i], rays6[6 * i + 1], rays6[6 * i + 2]},
-                         v3{rays6[6 * i + 3], rays6[6 * i + 4], rays6[6 * i + 5]});
+        const float *r = rays6 + record_at(i, 6);
+        trav_begin_scene(sv, s, v3{r[0], r[1], r[2]}, v3{r[3], r[4], r[5]});
         return S.instCount > 0;
     };
     auto store = [&](uint32_t i, const Trav &s) {
         const SceneHit &h = s.out;
-        float *r = out7 + 7 * (size_t)i;
+        float *r = out7 + record_at(i, 7);
         if (h.inst == SPG_MISS)
         {
             r[0] = -1.0f;
