@@ -194,7 +194,7 @@ def bench_config1(args, V, scenes):
     for _ in range(args.warmup):
         V.path_trace_tiles_device(ctx, tiles, img)
     dev.synchronize()
-    ext_ms, ext_n, steps_ms = 0.0, 0, []
+    ext_ms, ext_n, tot_ms, steps_ms = 0.0, 0, 0.0, []
     t0 = time.perf_counter()
     for _ in range(args.steps):
         ts = time.perf_counter()
@@ -203,6 +203,7 @@ def bench_config1(args, V, scenes):
         tim = dev.last_timings()
         ext_ms += tim["extend"][0]
         ext_n += tim["extend"][1]
+        tot_ms += tim["total"][0]
     dev.synchronize()
     wall = time.perf_counter() - t0
     # counting run of the same launches: slab and triangle tests, rays
@@ -237,7 +238,7 @@ def bench_config1(args, V, scenes):
                      "launch_ms": mean_ms, "algorithmic_bytes_per_launch": per_launch_bytes,
                      "rays_per_step": rays, "slab_tests_per_ray": box / max(rays, 1),
                      "tri_tests_per_ray": tri / max(rays, 1)},
-        "extra": {"gpu_ms_per_step": dev.last_timings()["total"][0],
+        "extra": {"gpu_ms_per_step": tot_ms / args.steps,
                   "Mrays_per_s": rays * args.steps / wall / 1e6,
                   "step_ms": steps_ms},
     }
@@ -362,6 +363,7 @@ def bench_box(args, V, scenes, name):
     per_launch = bytes_step / launches
     mean_ms = ext_ms / ext_n
     achieved = per_launch / (mean_ms * 1e-3) / 1e9
+    counted = name == "config5" and est == V.EST_UNBIASED   # the counter runs' launches
     samples = w * h * spp
     res = {
         "metric": METRIC,
@@ -383,16 +385,16 @@ def bench_box(args, V, scenes, name):
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": (TRAFFIC_BYTES_PER_RAY["config5"] * rays / launches
-                                 if name == "config5" else None),
-                     "traffic_source": TRAFFIC_SOURCE if name == "config5" else None,
+                                 if counted else None),
+                     "traffic_source": TRAFFIC_SOURCE if counted else None,
                      "traffic_frac": (TRAFFIC_BYTES_PER_RAY["config5"] * rays / launches /
                                       (mean_ms * 1e-3) / 1e9 / HBM_PEAK_GBS
-                                      if name == "config5" else None),
+                                      if counted else None),
                      "kernel": "k_extend (closest-hit traversal)",
                      "launch_ms": mean_ms, "algorithmic_bytes_per_launch": per_launch,
                      "compulsory_bytes_per_launch": (RAY_BYTES + HIT_BYTES_SCENE) * rays /
                      launches + scene_bytes,
-                     "limiter": LIMITER.get(name),
+                     "limiter": LIMITER.get(name) if counted else None,
                      "rays_per_step": rays, "slab_tests_per_ray": box / max(rays, 1),
                      "tri_tests_per_ray": tri / max(rays, 1),
                      "tlas_slab_tests_per_ray": tbox / max(rays, 1),
