@@ -592,7 +592,8 @@ int spg_obj_parse(const char *text, size_t len, float *verts8, uint32_t vertCap,
  * RGBA32F texels (host memory, face-major like HdrCubeMap.images).
  * transcendentals: SPG_TX_DOUBLE (sums bit-identical to the oracle's
  * double-evaluated restatement) or SPG_TX_FAST.  kernelMs (may be NULL)
- * receives the kernel's time. */
+ * receives the kernel's time.  The device keeps the call's buffer (source
+ * and faces) for the next one, up to 64 MB, until it is destroyed. */
 int spg_create_irradiance_cubemap(spg_Device *dev, const float *equirect,
                                   uint32_t ew, uint32_t eh, uint32_t faceWidth,
                                   uint32_t faceHeight, float radianceClamp,

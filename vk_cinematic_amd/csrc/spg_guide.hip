@@ -460,9 +460,11 @@ hipError_t launch_guide_gradient(hipStream_t s, const GuideTrainArgs &a,
 
 // Four launches: each small one costs about 4.4 us, so the loss's clear and
 // the step count ride on the weight sum and the gradient's sum on the update
-// (seven launches before).  k_guide_fwdbwd, batch 16384: 19.7 -> 11 us with
-// the staging's loads in flight together; 2 or 1 waves per block instead of 4
-// wait longer for the staging (29.7 and 50 us before that change).
+// (seven launches before).  k_guide_fwdbwd with the staging's loads in flight
+// together: full batches of 16,384 samples 41.0 -> 33.0 us; over the steps of a
+// 512 x 512 training call, most of whose batches are partly empty, 19.7 -> 11 us
+// on average.  On those steps 2 or 1 waves per block instead of 4 waited longer
+// for the staging (29.7 and 50 us, measured before that change).
 hipError_t launch_guide_train_step(hipStream_t s, const GuideTrainArgs &a,
                                    const GuideAdam &h, uint32_t cus)
 {

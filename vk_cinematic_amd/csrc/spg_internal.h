@@ -163,7 +163,7 @@ struct DevPaths
     uint64_t *rngPcg;            // PCG state per path
     uint32_t *slotRng;           // xorshift state carried per pixel slot
     float *vtx;                  // [bounces*7][capacity]: E.xyz X.xyz cos
-    uint32_t *vcount;            // vertices per path
+    uint32_t *vcount;            // vertices of a finished path (parity, guided)
     float *beta;                 // [3][capacity]
     float *radiance;             // [3][capacity]
     float *qo[3], *qd[3];        // [3][capacity] ray origins / directions

@@ -81,7 +81,7 @@ __device__ __forceinline__ h8 pack_tiles(f4 a, f4 b)
 // Copy fp16 rows of 64 (global, 16-byte aligned) into LDS rows of kLdsPitch,
 // whole block.  Eight 16-byte loads of a thread are in flight together: with
 // one 8-byte load per iteration a 256-thread block waited for 40 round trips
-// before its first product (k_guide_fwdbwd 19.7 -> 11 us).
+// before its first product (k_guide_fwdbwd 41.0 -> 33.0 us for 16,384 samples).
 __device__ __forceinline__ void stage_rows(_Float16 *dst, const _Float16 *src,
                                            int rows)
 {

@@ -8,7 +8,7 @@
 //                                  local ray -> BLAS (sp_RayIntersectScene)
 //   wavefront     k_raygen -> (k_extend -> k_shade)* -> k_finalize
 //                 rays live in SoA queues; k_shade appends continuing rays
-//                 to the next queue with a wave ballot + one atomic per wave
+//                 to the next queue with a wave ballot + one atomic per block
 //
 // All arithmetic that the reference defines is written in its operation
 // order (spg_math.h) and built with -ffp-contract=off and correctly rounded
@@ -1010,17 +1010,18 @@ __device__ __forceinline__ float nee_hit_weight(const TraceParams &p, const DevS
 
 // One bounce of every queued path: surface, material, scatter, vertex record
 // (parity) or throughput update (unbiased), append continuing rays to queue
-// q^1 with a ballot + one atomic per wave.
+// q^1 with a ballot + one atomic per block.
 //
 // Bound by the latency of its reads (state, then the hit's triangle and
-// material) at the two waves per SIMD that the double-precision
-// transcendentals leave (182 registers; budgets for three to five waves
-// spill: a 1080p pass's 955 us become 924, 1172, 1438, next-event
-// estimation's 602 become 653, 704, 815).  So it moves only state that is
-// read again: a path's vertex
-// count is the bounce, its throughput and radiance start from constants, and
-// a finished path keeps no throughput, stream or (unbiased) count (1080p room,
-// 6 bounces, 955 -> 843 us).
+// material) at the few waves per SIMD that the registers of the
+// double-precision transcendentals leave.  So it moves only state that is read
+// again: a path's vertex count is the bounce, its throughput and radiance start
+// from constants, and a finished path keeps no throughput, stream or (unbiased)
+// count (1080p room, 6 bounces, 955 -> 843 us; it also took the unbiased kernel
+// from two waves per SIMD to three, 166 registers; next-event estimation: 182
+// and 68 bytes of spill, two waves).  Register budgets for three, four and five waves, measured before
+// that change: unbiased 955 -> 924, 1172 and 1438 us, next-event estimation 602
+// -> 653, 704 and 815 (spills), so no budget is set.
 template <bool kDouble, int kEst, bool kBatch>
 __global__ __launch_bounds__(256) void k_shade(TraceParams p, int q)
 {
@@ -1762,7 +1763,8 @@ __global__ void k_set_u32(uint32_t *p, uint32_t v) { *p = v; }
 // The mesh walk is bound by its node and triangle fetches (random rays
 // share few of them): more resident waves evict each other's lines from the
 // CU's 32 KB L1.  2^21 rays on 500k triangles: 8 waves per CU 516 us, 10
-// 513, 12 530; 300k rays on 100k triangles 264, 247, 243.
+// 513, 12 530; 300k rays on 100k triangles 264, 247, 243 (12 gains 1.6%
+// there and costs the larger list 3%).
 constexpr uint32_t kMeshWavesPerCU = 10;
 
 hipError_t launch_closest_mesh(hipStream_t s, const DevMesh *mesh,

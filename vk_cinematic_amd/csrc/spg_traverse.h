@@ -9,7 +9,8 @@
 // t).  The walk is bound by vector instruction issue, and a wave pays for a
 // kind's instructions whether one of its lanes or all 64 are of that kind:
 // with every kind run in every iteration the 4M-triangle room took 253
-// instructions per ray at 22% of the lanes busy (now 172).  So an iteration
+// instructions per ray (now 172), about five times what its steps are with all
+// lanes busy.  So an iteration
 // runs ONE kind, the one that most lanes wait for (persistent_walk), and
 // the other lanes keep their state; what a lane does, and in which order,
 // does not depend on it.  A hit leaf child becomes the lane's leaf range
@@ -25,7 +26,7 @@
 // Measured against all kinds per iteration, per pass: 1M-triangle box scene
 // at 512x512 2397 -> 1757 us, 4M-triangle room at 1080p 5443 -> 4415,
 // 1M-triangle room with shadow rays 3979 -> 2784, 256x256 frame 361 -> 200,
-// 64x64 tile 110 -> 74; mesh rays: 2^21 on 500k triangles 664 -> 516.
+// 64x64 tile 110 -> 74; mesh rays: 2^21 on 500k triangles 664 -> 513.
 //
 // Stack: the top entries of each lane live in LDS (4 or 8 KB per wave);
 // deeper entries spill to a global array (rare: the builder bounds
@@ -48,6 +49,11 @@ constexpr uint32_t kSceneChunk = 128, kMeshChunk = 128;
 // that waits for a rare kind costs as much as one that waits for a node, but
 // the node step is the longest (about 150 instructions against 60 to 90),
 // and a rare kind that waits until it has the most lanes waits for long.
+// Box at 512x512, room at 1080p and room with shadow rays, us per call: equal
+// weights 2182, 5540, 3688; 1 2 2 2 2111, 5348, 3470; 1 3 3 3 2139, 5438,
+// 3541; 1 2 4 6 2107, 5428, 3494; 2 3 4 5 2091, 5319, 3461; these 2104, 5384,
+// 3492, so the weights have to differ but within 1.5% it does not matter how.
+// Mesh rays (2^21 on 500k triangles): 1 1 554, 2 3 530, 1 3 524, 1 2 524.
 constexpr int kNodeWeight = 1, kTriangleWeight = 2, kEnterWeight = 3, kFinishWeight = 4;
 
 // Node, triangle and stack-spill arrays are reached through pointers read
